@@ -87,6 +87,11 @@ SIGNATURES = {
     "gs_render_bwd": (
         ctypes.c_int, [_i32, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp],
     ),
+    "gs_render_bwd_workspace_bytes": (_sz, [_i32, _i32, _i32, _i64]),
+    "gs_render_bwd_ws": (
+        ctypes.c_int,
+        [_i32, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz, _vp],
+    ),
     "gs_preprocess_bwd": (
         ctypes.c_int,
         [_i32, _i32, _i32, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _f32, _f32, _f32, _f32, _vp, _vp, _vp, _vp,

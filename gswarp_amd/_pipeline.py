@@ -762,12 +762,14 @@ def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, gra
             gd = _f32c_or_none(grad_depth)
             ga = _f32c_or_none(grad_alpha)
             alpha_c = _f32c(alpha)
+            ws_bytes = int(lib.gs_render_bwd_workspace_bytes(W, H, P, bins.num_rendered))
+            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=device) if ws_bytes > 0 else None
             with _stage("render_bwd"):
-                lib.call("gs_render_bwd", W, H, P, bins.num_rendered, bins.ranges.data_ptr(),
+                lib.call("gs_render_bwd_ws", W, H, P, bins.num_rendered, bins.ranges.data_ptr(),
                          bins.point_list.data_ptr(), pre.records.data_ptr(), bg.data_ptr(), alpha_c.data_ptr(),
                          n_contrib.data_ptr(), _lib.ptr(gc), _lib.ptr(gd), _lib.ptr(ga),
                          int(bool(options.compute_depth)), grad_gauss.data_ptr(), _lib.ptr(bins.tile_order),
-                         stream)
+                         _lib.ptr(ws), ws_bytes, stream)
         has_sh = inputs.sh.numel() != 0
         shs = _f32c(inputs.sh).reshape(P, -1, NUM_CHANNELS) if has_sh else None
         K = shs.shape[1] if has_sh else 0

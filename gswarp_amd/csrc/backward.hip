@@ -242,6 +242,22 @@ struct RenderBwdParams {
   const int* tile_order;  // the tiles in the order the workgroups take them (gs_tile_order), null: tile order
 };
 
+// A part of a slice's walk (render_bwd_segment): the list positions [lo, hi).
+// The state (1/T, S) of a pixel changes over a segment by
+//   1/T <- a (1/T),  S <- b + a S,
+// with a the product of (1 - alpha) over the segment and b the S that the
+// segment gives a pixel starting from 0.  kCompose walks a segment for that
+// map alone (no gradients); kGradients starts from the pixel's state at the
+// list's end and the maps of the segments behind its own.
+enum class SegmentMode { kWhole, kCompose, kGradients };
+
+struct WalkSegment {
+  int lo = 0, hi = 0;
+  int behind = 0;                // segments behind this one
+  const float2* maps = nullptr;  // their (a, b), 64 kPix each, nearest first
+  float2* map_out = nullptr;     // kCompose: this segment's
+};
+
 // One wave walks a slice of kPix blocks of 8x8 pixels, kCols blocks wide:
 // lane l owns pixel (l % 8, l / 8) of every block, block k lying at
 // ((k % kCols) 8, (k / kCols) 8) from the slice's origin.  Slice `sub` of a
@@ -282,9 +298,9 @@ struct RenderBwdParams {
 // a visit classifies a pixel with two unsigned compares of q's bits.
 // s_rec (3 x 64 float4) and s_slot (kSlotLdsFloats floats, 16-byte aligned)
 // are the wave's LDS.
-template <bool kDepth, int kPix, int kCols, bool kBlockCull>
+template <bool kDepth, int kPix, int kCols, bool kBlockCull, SegmentMode kSegment = SegmentMode::kWhole>
 __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int tile, int sub, float4* s_rec,
-                                                 float* s_slot) {
+                                                 float* s_slot, WalkSegment seg = WalkSegment()) {
   static_assert(kPix % kCols == 0 && 8 * kCols <= kBlockX && 8 * (kPix / kCols) <= kBlockY, "slice in a tile");
   constexpr int kSliceW = 8 * kCols;
   constexpr int kSliceH = 8 * (kPix / kCols);
@@ -347,8 +363,31 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
     S[k] = live ? fmaf(bg2, gp2[k], fmaf(bg1, gp1[k], bg0 * gp0[k])) : 0.0f;
     lmax = imax(lmax, last[k]);
   }
-  const int max_lc = __builtin_amdgcn_readfirstlane(wave_max_i32(lmax));
-  if (max_lc == 0) return;
+  // The walk's list positions: [lo, max_lc), back to front.
+  int max_lc = __builtin_amdgcn_readfirstlane(wave_max_i32(lmax));
+  int lo = 0;
+  if constexpr (kSegment != SegmentMode::kWhole) {
+    lo = seg.lo;
+    max_lc = imin(max_lc, seg.hi);
+    if constexpr (kSegment == SegmentMode::kCompose) {
+#pragma unroll
+      for (int k = 0; k < kPix; ++k) {
+        Ti[k] = 1.0f;
+        S[k] = 0.0f;
+      }
+    } else {
+      // the pixels' state behind the segment: the segments behind it, applied in turn
+      for (int s = seg.behind - 1; s >= 0; --s) {
+#pragma unroll
+        for (int k = 0; k < kPix; ++k) {
+          const float2 ab = seg.maps[(s * kPix + k) * 64 + lane];
+          Ti[k] *= ab.x;
+          S[k] = fmaf(ab.x, S[k], ab.y);
+        }
+      }
+    }
+  }
+  if (max_lc <= lo) return;
   const int flush_comp = lane < kSlotFloats / 4 ? slot_component(lane >> 2) : -1;  // kCols == 2
   float* const col_raw = s_slot + kColSlotFloats;  // kCols == 1: the column slot, then the sums
   const int raw_ofs = col_raw_offset(lane);
@@ -366,11 +405,11 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
   // which leaves the compiler nothing to merge, and so nothing to wait for,
   // right after them.
   const int* const list = p.point_list + rg.x;
-  int bs = imax(0, max_lc - 64);
+  int bs = imax(lo, max_lc - 64);
   int id = checked_point(batch_entry(list, bs, max_lc - bs, max_lc, lane), p.num_points);
-  int id_ahead = batch_entry(list, imax(0, bs - 64), bs - imax(0, bs - 64), max_lc, lane);
+  int id_ahead = batch_entry(list, imax(lo, bs - 64), bs - imax(lo, bs - 64), max_lc, lane);
   RecordRegs next = load_record(p.records, id);
-  for (int batch_end = max_lc; batch_end > 0; batch_end = bs, bs = imax(0, bs - 64)) {
+  for (int batch_end = max_lc; batch_end > lo; batch_end = bs, bs = imax(lo, bs - 64)) {
     const int cnt = batch_end - bs;
     // One wave per workgroup: its LDS queue orders these writes before the
     // broadcast reads below.  In the LDS copy r1.w (qcut, which the visits
@@ -411,7 +450,7 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
     // the next batch [bs - 64, bs): its records; and the indices of the one
     // after it (either may be empty: the loads then read a valid entry)
     {
-      const int nbs = imax(0, bs - 64), nnbs = imax(0, nbs - 64);
+      const int nbs = imax(lo, bs - 64), nnbs = imax(lo, nbs - 64);
       id = checked_point(id_ahead, p.num_points);
       next = load_record(p.records, id);
       id_ahead = batch_entry(list, nnbs, nbs - nnbs, max_lc, lane);
@@ -513,10 +552,15 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
           // 1/T in front of this Gaussian: (1/T behind it) (1 - alpha), with
           // 1 - alpha >= 1 - kAlphaMax (the reference's 1e-5 floor never applies)
           const float tin = fmaf(-alpha, Ti[k], Ti[k]);
-          const float Tn = __builtin_amdgcn_rcpf(tin);
           float fu = fmaf(f.z, gp2[k], fmaf(f.y, gp1[k], fmaf(f.x, gp0[k], gpa[k])));
           if (kDepth) fu = fmaf(b.z, gpd[k], fu);
           const float d = fu - S[k];
+          if constexpr (kSegment == SegmentMode::kCompose) {
+            S[k] = fmaf(alpha, d, S[k]);
+            Ti[k] = tin;
+            return;
+          }
+          const float Tn = __builtin_amdgcn_rcpf(tin);
           const float v = G * (Tn * d);
           const float dch = alpha * Tn;
           const float vdy = v * dy[k];
@@ -541,6 +585,7 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
 #pragma unroll
         for (int k = 0; k < kPix; ++k)
           if (cand_lanes[k] != 0) blend(k);
+        if constexpr (kSegment == SegmentMode::kCompose) continue;
         // Pixel moments of v about the Gaussian's mean; the conic, opacity
         // and W/2, H/2 factors are per Gaussian and applied once, when the
         // per-Gaussian backward turns the sums into 2D gradients.
@@ -604,6 +649,11 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
       walk(std::true_type{});
     else
       walk(std::false_type{});
+  }
+  if constexpr (kSegment == SegmentMode::kCompose) {
+#pragma unroll
+    for (int k = 0; k < kPix; ++k) seg.map_out[64 * k + lane] = make_float2(Ti[k], S[k]);
+    return;
   }
   if (slot_gid >= 0) {
     if constexpr (kCols == 1)
@@ -671,6 +721,157 @@ __global__ __launch_bounds__(64, 6) void render_bwd_kernel(RenderBwdParams p) {
 template <bool kDepth>
 __global__ __launch_bounds__(64) void render_bwd_whole_kernel(RenderBwdParams p) {
   render_bwd_tiles<kDepth, true>(p);
+}
+
+// The walk in segments.  On images of few tiles the slices of render_bwd_tiles
+// leave most of the chip idle, and the kernel lasts as long as its longest
+// serial walk (about 0.25 us an entry).  Here the walk of a slice (quadrants,
+// kPix 1, or halves, kPix 2) of L entries is cut into min(max_segments,
+// ceil(L / kSegmentEntries)) segments of equal length, each walked by a wave
+// of its own, after a first launch has walked every segment but the front
+// ones for its map (SegmentMode).  slice_walk_kernel finds every slice's L,
+// so that the waves of segments that do not exist return on one load.
+//
+// Kernel times of the three launches against the unsegmented walk, us:
+// 1M Gaussians on 640x640 (4.6k entries on a few tiles) 1605 -> 190, 262k on
+// 384x384 683 -> 100, 100k on 800x800 160 -> 92, 300k on 800x800 245 -> 165,
+// 60k on 487x273 106 -> 50.  Segments of 256 entries: 115 and 62 for the third
+// and the last.  Walking the last segments' gradients in the first launch,
+// which saves their maps, measured the same.
+constexpr int kSegmentEntries = 128;
+
+// Most segments of a walk: more where there are fewer tiles, since each
+// costs a wave per slice that returns at once when its walk is shorter (about
+// 1.5 us per 10,000).  640x640: 16 segments 182 us, 8 207 us; 800x800, 300k
+// Gaussians: 8 segments 156 us, 16 176 us.
+static int max_segments(int64_t num_tiles) { return num_tiles <= 1024 ? 32 : num_tiles <= 2048 ? 16 : 8; }
+
+// Entries per segment (a multiple of 64, whole batches) of a walk.
+__device__ __forceinline__ int segment_length(int walk, int max_segments) {
+  const int count = imin(max_segments, (walk + kSegmentEntries - 1) / kSegmentEntries);
+  return count <= 1 ? walk : ((walk + count - 1) / count + 63) & ~63;
+}
+
+// walk[kSubs tile + sub]: the largest n_contrib of the slice's pixels, at
+// most the length of the tile's list.
+template <int kPix>
+__global__ __launch_bounds__(256) void slice_walk_kernel(RenderBwdParams p, int* __restrict__ walk) {
+  constexpr int kSubs = 4 / kPix;
+  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (unit >= kSubs * p.num_tiles) return;
+  const int lane = threadIdx.x & 63;
+  const int tile = unit / kSubs, sub = unit % kSubs;
+  const int x = (tile % p.grid_x) * kBlockX + (sub & 1) * 8 + (lane & 7);
+  const int y0 = (tile / p.grid_x) * kBlockY + (sub >> 1) * 8 + (lane >> 3);
+  int2 rg = p.ranges[tile];
+  int last = 0;
+#pragma unroll
+  for (int k = 0; k < kPix; ++k) {
+    const int y = y0 + 8 * k;
+    const int n = p.n_contrib[imin(y, p.H - 1) * p.W + imin(x, p.W - 1)];
+    if (x < p.W && y < p.H) last = imax(last, n);
+  }
+  rg.x = imax(0, imin(rg.x, p.num_rendered));
+  rg.y = imax(rg.x, imin(rg.y, p.num_rendered));
+  last = wave_max_i32(imin(last, rg.y - rg.x));
+  if (lane == 0) walk[unit] = last;
+}
+
+// Workgroup b: segment b / units (the one after it when composing) of
+// slice b % units, units = xcd_grid(kSubs num_tiles).  maps holds 64 kPix
+// (a, b) for each of a slice's max_segments - 1 segments behind its front
+// one.
+template <bool kDepth, int kPix, bool kCompose>
+__device__ __forceinline__ void render_bwd_segment(const RenderBwdParams& p, const int* walk, float2* maps,
+                                                   int max_segments, float4* s_rec, float* s_slot) {
+  constexpr int kSubs = 4 / kPix;
+  const int units = xcd_grid(kSubs * p.num_tiles);
+  const int unit = xcd_unit(blockIdx.x % units, kSubs * p.num_tiles);
+  if (unit >= kSubs * p.num_tiles) return;
+  const int index = blockIdx.x / units + (kCompose ? 1 : 0);
+  const int length = walk[unit];
+  const int step = segment_length(length, max_segments);
+  WalkSegment seg;
+  seg.lo = index * step;
+  if (seg.lo >= length) return;
+  seg.hi = imin(seg.lo + step, length);
+  seg.behind = (length + step - 1) / step - 1 - index;
+  float2* const own = maps + ((size_t)unit * (max_segments - 1) + index) * (64 * kPix);
+  seg.maps = own;  // of segment index + 1 and on
+  if constexpr (kCompose) seg.map_out = own - 64 * kPix;
+  render_bwd_slice<kDepth, kPix, 1, false, kCompose ? SegmentMode::kCompose : SegmentMode::kGradients>(
+      p, unit / kSubs, unit % kSubs, s_rec, s_slot, seg);
+}
+
+template <bool kDepth, int kPix>
+__global__ __launch_bounds__(64) void render_bwd_compose_kernel(RenderBwdParams p, const int* __restrict__ walk,
+                                                                float2* __restrict__ maps, int max_segments) {
+  __shared__ float4 s_rec[3 * 64];
+  render_bwd_segment<kDepth, kPix, true>(p, walk, maps, max_segments, s_rec, nullptr);
+}
+
+template <bool kDepth, int kPix>
+__global__ __launch_bounds__(64, 6) void render_bwd_segments_kernel(RenderBwdParams p, const int* __restrict__ walk,
+                                                                    float2* __restrict__ maps, int max_segments) {
+  __shared__ float4 s_rec[3 * 64];
+  __shared__ __align__(16) float s_slot[kColSlotFloats + kColRawFloats];
+  render_bwd_segment<kDepth, kPix, false>(p, walk, maps, max_segments, s_rec, s_slot);
+}
+
+// Pixels per lane of the segmented walk, or 0 for render_bwd_tiles.  All times
+// are the kernels' sums in us, unsegmented / halves / quadrants in segments.
+// - Above 2600 tiles the unsegmented waves fill the chip (300k Gaussians on
+//   1280x720, 3600 tiles: 176 / 184 / 189).
+// - Above 12 pairs per Gaussian the large splats' rows of grad_gauss are
+//   contended, and every further slice adds flushes to them: halves, and only
+//   up to 1600 tiles (a tenth of the splats large, 640x480: 93 / 79 / 123,
+//   800x600: 98 / 104 / 189).
+// - Else quadrants up to 1600 tiles (1M on 640x480: 374 / 258 / 257, 300k on
+//   400x300: 523 / 209 / 136) and for 4 to 12 pairs per Gaussian (100k
+//   mid-sized splats on 680x680: 316 / 132 / 125).
+// - Between, by the work: quadrants up to 500k pairs (100k on 800x800:
+//   160 / 129 / 92), halves up to 1.25M (300k on 800x800: 245 / 165 / 156, 600k:
+//   347 / 254 / 253, 1000x500: 191 / 194 / 209), unsegmented beyond (1M on
+//   960x640, 1.7M pairs: 299 / 327 / 334).
+constexpr int64_t kSegmentContendedPairsPerPoint = 12;
+
+static int segment_pixels(int64_t num_tiles, int64_t num_rendered, int64_t num_points) {
+  if (num_tiles > 2600) return 0;
+  if (num_rendered > kSegmentContendedPairsPerPoint * num_points) return num_tiles <= 1600 ? 2 : 0;
+  if (num_tiles <= 1600 || num_rendered > kWholeTilePairsPerPoint * num_points) return 1;
+  return num_rendered <= 500000 ? 1 : num_rendered <= 1250000 ? 2 : 0;
+}
+
+// The workspace of the segmented walk: the maps of every quadrant (or, at
+// two pixels per lane, half), then the walk lengths.
+static size_t segment_maps_bytes(int64_t num_tiles) {
+  return (size_t)num_tiles * (max_segments(num_tiles) - 1) * kTilePixels * sizeof(float2);
+}
+
+static size_t segment_workspace_bytes(int64_t num_tiles) {
+  return segment_maps_bytes(num_tiles) + (size_t)num_tiles * 4 * sizeof(int);
+}
+
+template <bool kDepth, int kPix>
+static void launch_render_bwd_segments(const RenderBwdParams& p, char* workspace, hipStream_t s) {
+  constexpr int kSubs = 4 / kPix;
+  float2* const maps = reinterpret_cast<float2*>(workspace);
+  int* const walk = reinterpret_cast<int*>(workspace + segment_maps_bytes(p.num_tiles));
+  const int units = xcd_grid(kSubs * p.num_tiles);
+  const int segments = max_segments(p.num_tiles);
+  hipLaunchKernelGGL((slice_walk_kernel<kPix>), dim3((kSubs * p.num_tiles + 3) / 4), dim3(256), 0, s, p, walk);
+  hipLaunchKernelGGL((render_bwd_compose_kernel<kDepth, kPix>), dim3(units * (segments - 1)), dim3(64), 0, s, p, walk,
+                     maps, segments);
+  hipLaunchKernelGGL((render_bwd_segments_kernel<kDepth, kPix>), dim3(units * segments), dim3(64), 0, s, p, walk,
+                     maps, segments);
+}
+
+template <bool kDepth>
+static void launch_render_bwd_segments(const RenderBwdParams& p, int pixels, char* workspace, hipStream_t s) {
+  if (pixels == 1)
+    launch_render_bwd_segments<kDepth, 1>(p, workspace, s);
+  else
+    launch_render_bwd_segments<kDepth, 2>(p, workspace, s);
 }
 
 struct PreprocessBwdParams {
@@ -1353,12 +1554,21 @@ __global__ __launch_bounds__(256) void preprocess_bwd_kernel(PreprocessBwdParams
 
 }  // namespace gs
 
-extern "C" int gs_render_bwd(int32_t image_width, int32_t image_height, int32_t num_points,
+extern "C" size_t gs_render_bwd_workspace_bytes(int32_t image_width, int32_t image_height, int32_t num_points,
+                                                int64_t num_rendered) {
+  if (image_width <= 0 || image_height <= 0 || num_points <= 0 || num_rendered <= 0) return 0;
+  const int64_t tiles = ((int64_t)(image_width + gs::kBlockX - 1) / gs::kBlockX) *
+                        ((image_height + gs::kBlockY - 1) / gs::kBlockY);
+  return gs::segment_pixels(tiles, num_rendered, num_points) ? gs::segment_workspace_bytes(tiles) : 0;
+}
+
+extern "C" int gs_render_bwd_ws(int32_t image_width, int32_t image_height, int32_t num_points,
                              int64_t num_rendered, const int32_t* ranges,
                              const int32_t* point_list, const float* records, const float* background,
                              const float* out_alpha, const int32_t* n_contrib, const float* grad_color,
                              const float* grad_depth, const float* grad_alpha, int32_t compute_depth,
-                             float* grad_gauss, const int32_t* tile_order, void* stream) {
+                             float* grad_gauss, const int32_t* tile_order, void* workspace,
+                                size_t workspace_bytes, void* stream) {
   if (image_width <= 0 || image_height <= 0 || (long long)image_width * image_height > 0x7fffffffLL)
     return GS_ERR_INVALID_ARGUMENT;
   if (num_points <= 0 || num_rendered < 0) return GS_ERR_INVALID_ARGUMENT;
@@ -1366,6 +1576,9 @@ extern "C" int gs_render_bwd(int32_t image_width, int32_t image_height, int32_t 
   if (!ranges || !point_list || !records || !background || !out_alpha || !n_contrib || !grad_gauss)
     return GS_ERR_INVALID_ARGUMENT;
   if (reinterpret_cast<uintptr_t>(records) & 15) return GS_ERR_MISALIGNED;
+  if (reinterpret_cast<uintptr_t>(workspace) & 7) return GS_ERR_MISALIGNED;
+  const size_t needed = gs_render_bwd_workspace_bytes(image_width, image_height, num_points, num_rendered);
+  if (workspace && workspace_bytes < needed) return GS_ERR_INVALID_ARGUMENT;
   gs::RenderBwdParams p;
   p.W = image_width;
   p.H = image_height;
@@ -1384,6 +1597,16 @@ extern "C" int gs_render_bwd(int32_t image_width, int32_t image_height, int32_t 
   p.grad_alpha = grad_alpha;
   p.compute_depth = compute_depth;
   p.grad_gauss = grad_gauss;
+  if (workspace && needed > 0) {
+    p.tile_order = nullptr;
+    p.long_tile = 0;
+    const int pixels = gs::segment_pixels(p.num_tiles, num_rendered, num_points);
+    if (compute_depth)
+      gs::launch_render_bwd_segments<true>(p, pixels, static_cast<char*>(workspace), (hipStream_t)stream);
+    else
+      gs::launch_render_bwd_segments<false>(p, pixels, static_cast<char*>(workspace), (hipStream_t)stream);
+    return gs_status_from_hip(hipGetLastError());
+  }
   // four times the mean list length: only tiles that dominate the walk
   const int64_t long_tile = gs::kLongTileFactor * num_rendered / p.num_tiles;
   p.long_tile = long_tile > 0x7fffffffLL ? 0x7fffffff : (int)long_tile;
@@ -1405,6 +1628,16 @@ extern "C" int gs_render_bwd(int32_t image_width, int32_t image_height, int32_t 
       hipLaunchKernelGGL((gs::render_bwd_kernel<false>), grid, dim3(64), 0, s, p);
   }
   return gs_status_from_hip(hipGetLastError());
+}
+
+extern "C" int gs_render_bwd(int32_t image_width, int32_t image_height, int32_t num_points, int64_t num_rendered,
+                             const int32_t* ranges, const int32_t* point_list, const float* records,
+                             const float* background, const float* out_alpha, const int32_t* n_contrib,
+                             const float* grad_color, const float* grad_depth, const float* grad_alpha,
+                             int32_t compute_depth, float* grad_gauss, const int32_t* tile_order, void* stream) {
+  return gs_render_bwd_ws(image_width, image_height, num_points, num_rendered, ranges, point_list, records,
+                          background, out_alpha, n_contrib, grad_color, grad_depth, grad_alpha, compute_depth,
+                          grad_gauss, tile_order, nullptr, 0, stream);
 }
 
 extern "C" int gs_preprocess_bwd(int32_t P, int32_t sh_coeffs, int32_t degree, const float* means3d,

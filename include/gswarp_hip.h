@@ -512,6 +512,23 @@ int gs_render_bwd(int32_t image_width, int32_t image_height, int32_t num_points,
                   float* grad_gauss, const int32_t* tile_order, void* stream);
 
 /*
+ * gs_render_bwd with a workspace (8-byte aligned, gs_render_bwd_workspace_bytes
+ * bytes; NULL, or 0 bytes asked: gs_render_bwd itself) in which images of few
+ * tiles have their walks cut into segments that run side by side.  The sums
+ * differ only by rounding.
+ * Replaces: backward_ops.py:183-290 with backward_kernels.py:539-707.
+ */
+size_t gs_render_bwd_workspace_bytes(int32_t image_width, int32_t image_height, int32_t num_points,
+                                     int64_t num_rendered);
+int gs_render_bwd_ws(int32_t image_width, int32_t image_height, int32_t num_points, int64_t num_rendered,
+                     const int32_t* ranges,
+                     const int32_t* point_list, const float* records, const float* background,
+                     const float* out_alpha, const int32_t* n_contrib, const float* grad_color,
+                     const float* grad_depth, const float* grad_alpha, int32_t compute_depth,
+                     float* grad_gauss, const int32_t* tile_order, void* workspace, size_t workspace_bytes,
+                     void* stream);
+
+/*
  * Fused per-Gaussian backward: SH colour backward (when shs != NULL), the
  * projected-mean and depth gradients, cov2D -> cov3D -> scale/rotation
  * gradients, and the accumulation into grad_means3d / grad_means2d (z = 0).
