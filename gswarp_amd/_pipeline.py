@@ -21,8 +21,8 @@ import torch
 from . import _lib, _packing, _workspace
 from ._coverage import kernel_mode
 from ._runtime import BINNING_SORT_MODES, ExecutionOptions
-from ._state import (BinningState, ForwardResult, ForwardState, KeyLayout, PreprocessOutputs, RenderImages,
-                     RenderStageResult)
+from ._state import (ArenaBinningState, ArenaForwardState, ArenaPreprocessOutputs, BinningState, ForwardResult,
+                     ForwardState, KeyLayout, PreprocessOutputs, RenderImages, RenderStageResult, StateArena)
 
 BLOCK_X = 16
 BLOCK_Y = 16
@@ -113,6 +113,26 @@ def _f32c(t: torch.Tensor, align16: bool = False) -> torch.Tensor:
     if align16 and t.numel() and t.data_ptr() % 16:
         t = t.clone()
     return t
+
+
+def _address(t: torch.Tensor, copies: list, align16: bool = False) -> int:
+    """Address of t as contiguous fp32; a converted copy (_f32c) is appended to
+    ``copies``, which the caller keeps until its launches are enqueued."""
+    if t.dtype is not torch.float32 or not t.is_contiguous() or (align16 and t.data_ptr() % 16):
+        t = _f32c(t, align16)
+        copies.append(t)
+    return t.data_ptr()
+
+
+def _address_or_none(t: torch.Tensor | None, copies: list) -> int | None:
+    return None if t is None else _address(t, copies)
+
+
+def _device_guard(device: torch.device):
+    """torch.cuda.device(device), or nothing when it is the current device already."""
+    if device.index is None or torch.cuda.current_device() == device.index:
+        return contextlib.nullcontext()
+    return torch.cuda.device(device)
 
 
 def _focal(size: int, tanfov: float) -> float:
@@ -407,7 +427,21 @@ def binning(pre: PreprocessOutputs, image_height: int, image_width: int, options
         _workspace.note_pairs(device, R)
         _note("num_rendered", R)
     entries, valid_points = (slot[2], slot[3]) if sized else (-1, 0)
-    buffer = None
+    return _bin_exact(pre, image_height, image_width, mode, offsets, R, depth_range, entries, valid_points,
+                      keep_keys=keep_keys, pack=pack, ranges=ranges)
+
+
+def _bin_exact(pre: PreprocessOutputs, image_height: int, image_width: int, mode: str, offsets: torch.Tensor, R: int,
+               depth_range: int, entries: int, valid_points: int, *, keep_keys: bool = False, pack: bool = False,
+               ranges: torch.Tensor | None = None) -> BinningState:
+    """The binning after the read-back, into buffers of exactly R pairs, in
+    the dataflow that the mode picks.  entries and valid_points: the bucketed
+    binning's sizes (entries -1 when the scan did not size it)."""
+    device = pre.radii.device
+    P = pre.radii.shape[0]
+    grid_x, grid_y = grid_dims(image_width, image_height)
+    T = grid_x * grid_y
+    buffer = point_list = None
     if pack:
         buffer, point_list, ranges = _packing.allocate_binning(R, T, device)
     if R == 0:
@@ -421,7 +455,7 @@ def binning(pre: PreprocessOutputs, image_height: int, image_width: int, options
                                 and R <= DEPTH_TILE_MIN_PAIRS_PER_GAUSSIAN * P):
         _note("binning_dataflow", "packed_key")
         bins = _binning_packed(pre, image_width, image_height, offsets, R, layout, keep_keys, point_list, ranges)
-    elif sized and 0 <= entries <= MAX_BINNING_PAIRS:
+    elif 0 <= entries <= MAX_BINNING_PAIRS:
         _note("binning_dataflow", "buckets")
         _note("bucket_entries", entries)
         _note("bucket_valid", valid_points)
@@ -535,8 +569,8 @@ def _binning_buckets(pre: PreprocessOutputs, image_width: int, image_height: int
     nbytes = int(lib.gs_bin_buckets_workspace_bytes(P, valid_points, entries, image_width, image_height))
     ws = torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=device)
     events = _stage_chain(("depth_sort", "bucket", "bucket_tiles"))
-    lib.call("gs_bin_buckets", P, valid_points, entries, R, pre.depths.data_ptr(), depth_min, depth_max,
-             pre.coverage.data_ptr(), _lib.ptr(pre.band_store), pre.records.data_ptr(), image_width, image_height,
+    lib.call("gs_bin_buckets", P, valid_points, entries, R, pre.address("depths"), depth_min, depth_max,
+             pre.address("coverage"), pre.address("band_store"), pre.address("records"), image_width, image_height,
              ws.data_ptr(), ws.numel(), ranges.data_ptr(), point_list.data_ptr(), events, stream)
     keys = None
     if keep_keys:  # tile << 32 | depth bits, for tests
@@ -651,8 +685,7 @@ def render(pre: PreprocessOutputs, bins: BinningState, background: torch.Tensor,
         return RenderStageResult(color, depth, alpha, n_contrib, aux)
     compute_depth = int(bool(options.compute_depth))
     stream = _stream(device)
-    if bins.tile_order is None:
-        bins.tile_order = tile_order_buffer(W, H, device)
+    bins.ensure_tile_order(bins.grid_x * bins.grid_y)
     if flow:
         if write_aux:
             aux = (torch.empty((k, H, W), dtype=torch.int32, device=device), torch.empty((k, H, W), **f),
@@ -660,18 +693,18 @@ def render(pre: PreprocessOutputs, bins: BinningState, background: torch.Tensor,
         else:
             aux = _empty_flow_aux(0, H, W, device)
         with _stage("render"):
-            lib.call("gs_render_fwd_flow", W, H, P, bins.num_rendered, bins.ranges.data_ptr(),
-                     bins.point_list.data_ptr(), pre.records.data_ptr(), bg.data_ptr(), compute_depth,
+            lib.call("gs_render_fwd_flow", W, H, P, bins.num_rendered, bins.address("ranges"),
+                     bins.point_list.data_ptr(), pre.address("records"), bg.data_ptr(), compute_depth,
                      int(write_aux), k, color.data_ptr(), depth.data_ptr(), alpha.data_ptr(), n_contrib.data_ptr(),
                      aux[0].data_ptr() if write_aux else None, aux[1].data_ptr() if write_aux else None,
-                     aux[2].data_ptr() if write_aux else None, bins.tile_order.data_ptr(), stream)
+                     aux[2].data_ptr() if write_aux else None, bins.address("tile_order"), stream)
     else:
         with _stage("render"):
-            lib.call("gs_render_fwd_clear", W, H, P, bins.num_rendered, bins.ranges.data_ptr(),
-                     bins.point_list.data_ptr(), pre.records.data_ptr(), bg.data_ptr(), compute_depth,
+            lib.call("gs_render_fwd_clear", W, H, P, bins.num_rendered, bins.address("ranges"),
+                     bins.point_list.data_ptr(), pre.address("records"), bg.data_ptr(), compute_depth,
                      color.data_ptr(), depth.data_ptr(), alpha.data_ptr(), n_contrib.data_ptr(),
                      _lib.ptr(grad_clear), 0 if grad_clear is None else grad_clear.numel(),
-                     bins.tile_order.data_ptr(), stream)
+                     bins.address("tile_order"), stream)
     return RenderStageResult(color, depth, alpha, n_contrib, aux)
 
 
@@ -685,10 +718,14 @@ def forward(inputs: RasterInputs, options: ExecutionOptions, *, flow: bool = Fal
     if means.ndim != 2 or means.shape[1] != 3:
         raise ValueError("means3D must have dimensions (num_points, 3)")
     device = means.device
-    with torch.cuda.device(device), _workspace.device_lock(device):
+    with _device_guard(device), _workspace.device_lock(device):
         if means.shape[0] == 0:
             k = (options.flow_topk if options.compute_flow_aux else 0) if flow else None
             return empty_forward(inputs, k)
+        if not pack:
+            result = _forward_arena(inputs, options, device, flow=flow, grad_buffer=grad_buffer)
+            if result is not None:
+                return result
         pre = preprocess(inputs, options, pack=pack)
         images = render_images(inputs.background, inputs.image_height, inputs.image_width, options, device)
         grad_gauss = torch.empty((means.shape[0], _lib.GS_GRAD_FLOATS), dtype=torch.float32,
@@ -711,6 +748,127 @@ def forward(inputs: RasterInputs, options: ExecutionOptions, *, flow: bool = Fal
         state=ForwardState(pre, bins, res.n_contrib, grad_gauss),
         aux=res.aux,
     )
+
+
+def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torch.device, *, flow: bool,
+                   grad_buffer: bool) -> ForwardResult | None:
+    """The typed forward's ordinary course, with as little host work as it
+    needs: the same stages and launches as preprocess, binning and render
+    above, but the arrays that only the stages and the backward read lie in
+    one allocation (StateArena) and are passed by address.  None, with
+    nothing launched, where it does not apply: stage timing, other scan or
+    sort choices, the device's first forward (no pair count to provision
+    for), and inputs that the general course refuses.
+
+    Passes that the host bounds (60k Gaussians, 487x273): rendering 180 ->
+    134 us, a training step 499 -> 434 (with the one-pass input checks)."""
+    mode = options.binning_sort_mode
+    if (STAGE_TIMER is not None or not SCAN_ONEPASS or PACKED_SORT != "segmented" or inputs.prefiltered
+            or (mode != "warp_depth_stable_tile" and mode != "warp_radix")):
+        return None
+    P = inputs.means3d.shape[0]
+    W, H = inputs.image_width, inputs.image_height
+    cov_count, colors, sh = inputs.cov3d_precomp.numel(), inputs.colors, inputs.sh
+    has_sr = inputs.scales.numel() != 0 and inputs.rotations.numel() != 0
+    has_colors = colors.numel() != 0
+    K = 0 if has_colors else sh.numel() // (3 * P)
+    if (cov_count != 0) == has_sr or cov_count not in (0, 6 * P) or (not has_colors and sh.numel() != 3 * P * K) \
+            or (not has_colors and K == 0) or inputs.background.device != device:
+        return None
+    last = _workspace.last_pairs(device)
+    heavy = mode == "warp_depth_stable_tile" and last > DEPTH_TILE_MIN_PAIRS_PER_GAUSSIAN * P
+    sized = buckets_expected(options, W, H, P, device)
+    capacity = 0 if heavy else _workspace.pair_capacity(device)
+    if capacity <= 0 and not sized:
+        return None
+
+    lib = _lib.load()
+    stream_object = torch.cuda.current_stream(device)
+    stream = stream_object.cuda_stream
+    grid_x, grid_y = grid_dims(W, H)
+    T = grid_x * grid_y
+    coverage_mode = int(kernel_mode(options.tile_coverage_mode))
+    f32, i32 = torch.float32, torch.int32
+    scan_bytes = int(lib.gs_scan_state_bytes(P))
+    spans = [("records", f32, (P, _lib.GS_RECORD_FLOATS), 48 * P), ("coverage", i32, (P, 4), 16 * P),
+             ("depths", f32, (P,), 4 * P), ("tiles_touched", i32, (P,), 4 * P),
+             ("clamped", torch.uint8, (P,), P), ("ranges", i32, (T, 2), 8 * T), ("tile_order", i32, (T,), 4 * T),
+             ("n_contrib", i32, (H * W,), 4 * H * W), ("info", torch.int64, (4,), 32),
+             ("scan_state", torch.int64, (scan_bytes // 8,), scan_bytes)]
+    if sized:
+        words = max(int(lib.gs_band_store_words(P)), 1)
+        spans.append(("band_store", i32, (words,), 4 * words))
+    arena = StateArena(spans, device)
+    radii = torch.empty((P,), dtype=i32, device=device)
+    proj_2d = torch.empty((P, 2), dtype=f32, device=device)
+    conic_2d = torch.empty((P, 3), dtype=f32, device=device)
+    conic_2d_inv = torch.empty((P, 3), dtype=f32, device=device)
+    pre = ArenaPreprocessOutputs(radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode, arena)
+    copies = []
+    tanfovx, tanfovy = float(inputs.tan_fovx), float(inputs.tan_fovy)
+    radii_at, records_at, tiles_at = radii.data_ptr(), arena.address("records"), arena.address("tiles_touched")
+    coverage_at, depths_at, inv_at = arena.address("coverage"), arena.address("depths"), conic_2d_inv.data_ptr()
+    scan_at, info_at = arena.address("scan_state"), arena.address("info")
+    lib.call(
+        "gs_preprocess_fwd", P, K, int(inputs.degree), _address(inputs.means3d, copies),
+        _address(inputs.scales, copies) if has_sr else None, _address(inputs.rotations, copies, True) if has_sr else None,
+        _address(inputs.cov3d_precomp, copies) if cov_count else None, float(inputs.scale_modifier), _address(inputs.opacities, copies),
+        None if has_colors else _address(sh, copies), _address(colors, copies) if has_colors else None, _address(inputs.viewmatrix, copies),
+        _address(inputs.projmatrix, copies), _address(inputs.campos, copies), tanfovx, tanfovy, _focal(W, tanfovx), _focal(H, tanfovy),
+        W, H, coverage_mode, float(inputs.filter_variance), radii_at, depths_at, proj_2d.data_ptr(),
+        conic_2d.data_ptr(), inv_at, tiles_at, coverage_at, records_at, arena.address("clamped"),
+        pre.address("band_store"), words if sized else 0, scan_at, scan_bytes, stream)
+    offsets = torch.empty((P,), dtype=i32, device=device)
+    lib.call("gs_scan_tiles_onepass", P, tiles_at, offsets.data_ptr(), info_at, scan_at, scan_bytes, int(sized),
+             SCAN_SPIN_LIMIT, stream)
+    slot = _workspace.readback_slot(device, stream_object)
+    # the outputs and the backward's accumulator, allocated while the GPU works
+    color = torch.empty((NUM_CHANNELS, H, W), dtype=f32, device=device)
+    depth = torch.empty((1, H, W), dtype=f32, device=device)
+    alpha = torch.empty((1, H, W), dtype=f32, device=device)
+    grad_gauss = torch.empty((P, _lib.GS_GRAD_FLOATS), dtype=f32, device=device) if grad_buffer else None
+    compute_depth = bool(options.compute_depth)
+    bins = None
+    if capacity > 0:
+        point_list = torch.empty((capacity,), dtype=i32, device=device)
+        ws_bytes = int(lib.gs_bin_packed_workspace_bytes(capacity))
+        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=device)
+        result = (ctypes.c_int64 * 6)()
+        background = None if flow else _address(inputs.background, copies)
+        lib.call("gs_readback_bin_packed", info_at, slot.address, slot.next_seq(), P, radii_at, records_at, inv_at,
+                 coverage_at, depths_at, offsets.data_ptr(), W, H, coverage_mode,
+                 DEPTH_TILE_MIN_PAIRS_PER_GAUSSIAN if mode == "warp_depth_stable_tile" else 0, capacity,
+                 ws.data_ptr(), ws_bytes, arena.address("ranges"), point_list.data_ptr(), background,
+                 0 if flow else int(compute_depth), None if flow else color.data_ptr(),
+                 None if flow else depth.data_ptr(), None if flow else alpha.data_ptr(),
+                 None if flow else arena.address("n_contrib"), None if flow else _lib.ptr(grad_gauss),
+                 0 if flow or grad_gauss is None else grad_gauss.numel(), None, result,
+                 None if flow else arena.address("tile_order"), stream)
+        R = validate_pair_count(result[0])
+        _workspace.note_pairs(device, R)
+        if result[4]:
+            layout = KeyLayout(result[1], result[2], result[3])
+            bins = ArenaBinningState(grid_x, grid_y, point_list[:R], R, layout, arena, bool(result[5]))
+        else:
+            depth_range = slot[1] & 0xFFFFFFFFFFFFFFFF
+            # declined: release the provisioned buffers before the exact-size binning allocates its own
+            del ws, result, point_list
+            if sized:  # the call read back two values only
+                lib.call("gs_info_readback", info_at, slot.address, slot.next_seq(), 4, stream)
+    else:
+        lib.call("gs_info_readback", info_at, slot.address, slot.next_seq(), 4, stream)
+        R = validate_pair_count(slot[0])
+        depth_range = slot[1] & 0xFFFFFFFFFFFFFFFF
+        _workspace.note_pairs(device, R)
+    if bins is None:
+        entries, valid_points = (slot[2], slot[3]) if sized else (-1, 0)
+        bins = _bin_exact(pre, H, W, mode, offsets, R, depth_range, entries, valid_points)
+    aux: tuple[torch.Tensor, ...] = ()
+    if flow or not bins.rendered:
+        images = RenderImages(_f32c(inputs.background), color, depth, alpha, arena.view("n_contrib"), compute_depth)
+        aux = render(pre, bins, inputs.background, H, W, options, flow=flow, images=images, grad_clear=grad_gauss).aux
+    return ForwardResult(R, color, depth, alpha, radii, proj_2d, conic_2d, conic_2d_inv,
+                         ArenaForwardState(pre, bins, arena, grad_gauss), aux)
 
 
 def _depths_or_none(pre: PreprocessOutputs) -> int | None:
@@ -741,57 +899,52 @@ def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, gra
         return (torch.zeros((0, 3), dtype=torch.float32, device=device), grad_colors,
                 torch.empty_like(inputs.opacities), torch.zeros_like(means), grad_cov3d,
                 torch.empty_like(inputs.sh), torch.zeros_like(inputs.scales), torch.zeros_like(inputs.rotations))
-    with torch.cuda.device(device), _workspace.device_lock(device):
+    with _device_guard(device), _workspace.device_lock(device):
         if forward_state is None:
             # Second backward of a retained graph: rebuild the forward state.
             pre = preprocess(inputs, options)
             bins = binning(pre, H, W, options)
             n_contrib = render(pre, bins, inputs.background, H, W, options).n_contrib
+            n_contrib_at = n_contrib.data_ptr()
         else:
-            pre, bins, n_contrib = forward_state.preprocess, forward_state.binning, forward_state.n_contrib
+            pre, bins, n_contrib_at = forward_state.preprocess, forward_state.binning, forward_state.address("n_contrib")
         stream = _stream(device)
+        copies = []  # converted inputs, alive until the launches are enqueued
+        f = dict(dtype=torch.float32, device=device)
         # the accumulator the forward render zeroed serves one backward
         grad_gauss = None if forward_state is None else forward_state.grad_gauss
         if grad_gauss is not None:
             forward_state.grad_gauss = None
         if grad_gauss is None or grad_gauss.shape[0] != P:
-            grad_gauss = torch.zeros((P, _lib.GS_GRAD_FLOATS), dtype=torch.float32, device=device)
+            grad_gauss = torch.zeros((P, _lib.GS_GRAD_FLOATS), **f)
+        grad_gauss_at, records_at = grad_gauss.data_ptr(), pre.address("records")
         if bins.num_rendered != 0:
-            bg = _f32c(inputs.background.to(device))
-            gc = _f32c_or_none(grad_color)
-            gd = _f32c_or_none(grad_depth)
-            ga = _f32c_or_none(grad_alpha)
-            alpha_c = _f32c(alpha)
             ws_bytes = int(lib.gs_render_bwd_workspace_bytes(W, H, P, bins.num_rendered))
             ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=device) if ws_bytes > 0 else None
             with _stage("render_bwd"):
-                lib.call("gs_render_bwd_ws", W, H, P, bins.num_rendered, bins.ranges.data_ptr(),
-                         bins.point_list.data_ptr(), pre.records.data_ptr(), bg.data_ptr(), alpha_c.data_ptr(),
-                         n_contrib.data_ptr(), _lib.ptr(gc), _lib.ptr(gd), _lib.ptr(ga),
-                         int(bool(options.compute_depth)), grad_gauss.data_ptr(), _lib.ptr(bins.tile_order),
-                         _lib.ptr(ws), ws_bytes, stream)
+                lib.call("gs_render_bwd_ws", W, H, P, bins.num_rendered, bins.address("ranges"),
+                         bins.address("point_list"), records_at, _address(inputs.background.to(device), copies),
+                         _address(alpha, copies), n_contrib_at, _address_or_none(grad_color, copies),
+                         _address_or_none(grad_depth, copies), _address_or_none(grad_alpha, copies),
+                         int(bool(options.compute_depth)), grad_gauss_at, bins.address("tile_order"), _lib.ptr(ws),
+                         ws_bytes, stream)
         has_sh = inputs.sh.numel() != 0
-        shs = _f32c(inputs.sh).reshape(P, -1, NUM_CHANNELS) if has_sh else None
-        K = shs.shape[1] if has_sh else 0
-        grad_sh = torch.empty((P, K, NUM_CHANNELS), dtype=torch.float32, device=device) if has_sh else \
-            torch.empty_like(inputs.sh)
-        f = dict(dtype=torch.float32, device=device)
+        K = inputs.sh.numel() // (3 * P) if has_sh else 0
+        grad_sh = torch.empty((P, K, NUM_CHANNELS), **f) if has_sh else torch.empty_like(inputs.sh)
         grad_means3d = torch.empty((P, 3), **f)
         grad_means2d = torch.empty((P, 3), **f)
-        scales_c, rot_c, cov_c = _covariance_inputs(inputs, P)
-        if cov_c is None:
-            grad_scales = torch.empty((P, 3), **f)
-            grad_rotations = torch.empty((P, 4), **f)
-        else:
+        has_cov = inputs.cov3d_precomp.numel() != 0
+        if has_cov:
+            if inputs.cov3d_precomp.numel() != 6 * P:
+                raise ValueError("cov3D_precomp must hold 6 values per Gaussian")
             # The precomputed-covariance branch of backward_ops.py:733-737.
             grad_scales = torch.zeros_like(inputs.scales)
             grad_rotations = torch.zeros_like(inputs.rotations)
             grad_cov3d = torch.empty((P, 6), **f)
+        else:
+            grad_scales = torch.empty((P, 3), **f)
+            grad_rotations = torch.empty((P, 4), **f)
         tanfovx, tanfovy = float(inputs.tan_fovx), float(inputs.tan_fovy)
-        means_c = _f32c(means)
-        campos_c = _f32c(inputs.campos)
-        view_c = _f32c(inputs.viewmatrix)
-        proj_c = _f32c(inputs.projmatrix)
         radii_c = radii.contiguous()
         # The opacity and colour gradients are columns 5 and 6-8 of grad_gauss
         # (the reference returns views of its render gradients,
@@ -799,23 +952,21 @@ def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, gra
         # that autograd does not copy a strided view into each leaf.
         grad_opacities = torch.empty((P,), **f)
         grad_colors_out = torch.empty((P, NUM_CHANNELS), **f) if inputs.colors.numel() != 0 else None
-        gp2 = _f32c_or_none(grad_proj_2d)
-        gcon = _f32c_or_none(grad_conic_2d)
-        gcov = _f32c_or_none(grad_conic_2d_inv)
         with _stage("preprocess_bwd"):
             lib.call(
-                "gs_preprocess_bwd", P, K, int(inputs.degree), means_c.data_ptr(), _lib.ptr(scales_c),
-                _lib.ptr(rot_c), _lib.ptr(cov_c), float(inputs.scale_modifier), _lib.ptr(shs), campos_c.data_ptr(),
-                view_c.data_ptr(), proj_c.data_ptr(), tanfovx, tanfovy, _focal(W, tanfovx), _focal(H, tanfovy),
-                radii_c.data_ptr(), pre.clamped.data_ptr(), grad_gauss.data_ptr(), pre.records.data_ptr(), W, H,
-                _lib.ptr(gp2), _lib.ptr(gcon),
-                _lib.ptr(gcov), int(bool(flow_double)), float(inputs.filter_variance), grad_means3d.data_ptr(),
-                grad_means2d.data_ptr(),
-                _lib.ptr(grad_scales) if cov_c is None else None,
-                _lib.ptr(grad_rotations) if cov_c is None else None,
-                _lib.ptr(grad_cov3d) if cov_c is not None else None,
-                grad_sh.data_ptr() if has_sh else None, grad_opacities.data_ptr(),
-                _lib.ptr(grad_colors_out), stream)
+                "gs_preprocess_bwd", P, K, int(inputs.degree), _address(means, copies),
+                None if has_cov else _address(inputs.scales, copies),
+                None if has_cov else _address(inputs.rotations, copies, True),
+                _address(inputs.cov3d_precomp, copies) if has_cov else None, float(inputs.scale_modifier),
+                _address(inputs.sh, copies) if has_sh else None, _address(inputs.campos, copies),
+                _address(inputs.viewmatrix, copies), _address(inputs.projmatrix, copies), tanfovx, tanfovy,
+                _focal(W, tanfovx), _focal(H, tanfovy), radii_c.data_ptr(), pre.address("clamped"), grad_gauss_at,
+                records_at, W, H, _address_or_none(grad_proj_2d, copies), _address_or_none(grad_conic_2d, copies),
+                _address_or_none(grad_conic_2d_inv, copies), int(bool(flow_double)), float(inputs.filter_variance),
+                grad_means3d.data_ptr(), grad_means2d.data_ptr(),
+                None if has_cov else grad_scales.data_ptr(), None if has_cov else grad_rotations.data_ptr(),
+                grad_cov3d.data_ptr() if has_cov else None, grad_sh.data_ptr() if has_sh else None,
+                grad_opacities.data_ptr(), _lib.ptr(grad_colors_out), stream)
     grad_opacities = grad_opacities.reshape(inputs.opacities.shape)
     if grad_colors_out is not None:
         grad_colors = grad_colors_out.reshape(inputs.colors.shape)

@@ -29,6 +29,10 @@ class PreprocessOutputs:
     # gs_scan_tiles_onepass state that the preprocess prepared (serves one scan), or None
     scan_state: torch.Tensor | None = None
 
+    def address(self, name: str) -> int | None:
+        tensor = getattr(self, name)
+        return None if tensor is None else tensor.data_ptr()
+
 
 @dataclass(slots=True)
 class KeyLayout:
@@ -70,6 +74,14 @@ class BinningState:
     rendered: bool = False  # the standard forward render was launched with the binning (RenderImages)
     tile_order: torch.Tensor | None = None  # (T,) int32 buffer the forward render was given (gs_tile_order)
 
+    def address(self, name: str) -> int | None:
+        tensor = getattr(self, name)
+        return None if tensor is None else tensor.data_ptr()
+
+    def ensure_tile_order(self, num_tiles: int) -> None:
+        if self.tile_order is None:
+            self.tile_order = torch.empty((max(num_tiles, 1),), dtype=torch.int32, device=self.ranges.device)
+
     def decode_keys(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
         """(tile id, depth float bits, sort field = tile and depth fields as one
         non-negative int64) of every sorted pair, from sorted_keys."""
@@ -98,6 +110,98 @@ class ForwardState:
     # (N, 10) float32 gradient accumulator that the forward render zeroed on
     # its way (None when the forward made none); one backward takes it
     grad_gauss: torch.Tensor | None = None
+
+    def address(self, name: str) -> int:
+        return getattr(self, name).data_ptr()
+
+
+class StateArena:
+    """One device allocation for the arrays that a typed forward keeps for its
+    backward and shows to nobody else.  The stages and the backward need
+    their addresses only; a tensor view is made when one is asked for, which
+    spares an allocation or a view of each on every call."""
+
+    __slots__ = ("buffer", "base", "spans")
+
+    def __init__(self, spans, device: torch.device):
+        """spans: (name, dtype, shape, bytes) of each array; every array starts on a 256-byte boundary."""
+        self.spans = {}
+        at = 0
+        for name, dtype, shape, nbytes in spans:
+            self.spans[name] = (at, dtype, shape, nbytes)
+            at += (nbytes + 255) & ~255
+        self.buffer = torch.empty((at,), dtype=torch.uint8, device=device)
+        self.base = self.buffer.data_ptr()
+
+    def address(self, name: str) -> int:
+        return self.base + self.spans[name][0]
+
+    def view(self, name: str) -> torch.Tensor:
+        at, dtype, shape, nbytes = self.spans[name]
+        return self.buffer[at:at + nbytes].view(dtype).view(shape)
+
+
+def _arena_field(name: str):
+    return property(lambda self: self.arena.view(name) if name in self.arena.spans else None)
+
+
+class ArenaPreprocessOutputs:
+    """PreprocessOutputs whose arrays, but for the four that the forward returns, lie in an arena."""
+
+    __slots__ = ("radii", "proj_2d", "conic_2d", "conic_2d_inv", "coverage_mode", "arena")
+    geom = None
+    scan_state = None  # the arena's state has served its scan
+    depths = _arena_field("depths")
+    tiles_touched = _arena_field("tiles_touched")
+    records = _arena_field("records")
+    clamped = _arena_field("clamped")
+    coverage = _arena_field("coverage")
+    band_store = _arena_field("band_store")
+
+    def __init__(self, radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode: int, arena: StateArena):
+        self.radii, self.proj_2d, self.conic_2d, self.conic_2d_inv = radii, proj_2d, conic_2d, conic_2d_inv
+        self.coverage_mode = coverage_mode
+        self.arena = arena
+
+    def address(self, name: str) -> int | None:
+        return self.arena.address(name) if name in self.arena.spans else None
+
+
+class ArenaBinningState(BinningState):
+    """BinningState of the packed binning launched with the read-back, its ranges and tile order in an arena."""
+
+    __slots__ = ("arena", "has_order")
+    ranges = _arena_field("ranges")
+    tile_order = property(lambda self: self.arena.view("tile_order") if self.has_order else None)
+
+    def __init__(self, grid_x, grid_y, point_list, num_rendered, key_layout, arena: StateArena, rendered: bool):
+        self.grid_x, self.grid_y = grid_x, grid_y
+        self.point_list, self.num_rendered, self.key_layout = point_list, num_rendered, key_layout
+        self.sorted_keys = self.buffer = None
+        self.arena, self.rendered, self.has_order = arena, rendered, rendered
+
+    def ensure_tile_order(self, num_tiles: int) -> None:
+        self.has_order = True
+
+    def address(self, name: str) -> int | None:
+        if name == "point_list":
+            return self.point_list.data_ptr()
+        if name == "tile_order" and not self.has_order:
+            return None
+        return self.arena.address(name)
+
+
+class ArenaForwardState:
+    """ForwardState with n_contrib in an arena."""
+
+    __slots__ = ("preprocess", "binning", "arena", "grad_gauss")
+    n_contrib = _arena_field("n_contrib")
+
+    def __init__(self, preprocess, binning, arena: StateArena, grad_gauss):
+        self.preprocess, self.binning, self.arena, self.grad_gauss = preprocess, binning, arena, grad_gauss
+
+    def address(self, name: str) -> int:
+        return self.arena.address(name)
 
 
 @dataclass(slots=True)
