@@ -385,6 +385,178 @@ __global__ __launch_bounds__(64) void render_fwd_kernel(RenderFwdParams p) {
   clear_share(p, lane);
 }
 
+// The forward in 4x4-pixel blocks: a wave walks a block of 16 pixels, four
+// records at a time.  Lane 4 i + g evaluates record g of the four at pixel i,
+// and each lane then blends all four in order: their alphas come from the
+// pixel's four lanes by DPP, every lane carries the pixel's transmittance and
+// weight sum, and lane g sums its channel (r, g, b, depth).  The serial chain
+// of a walk is a quarter as long as with one record a visit, and a block
+// meets fewer records than a quadrant.  Every value is formed by the
+// operations of render_fwd_tile in the same order, so the images are the
+// same bit for bit.
+//
+// A batch of 64 records is culled against the block and the records left are
+// written to LDS side by side, so that a step reads four neighbours.  A step
+// issues about 48 vector instructions for 64 evaluations, a visit of
+// render_fwd_tile 32, and a tile's records are loaded by 16 waves instead of
+// 4: at 1080p, where the issue rate binds, 391 us against 250.  Where the
+// longest walks bind (times in us, before and after): 10k Gaussians on
+// 256x256 32 and 12, 100k on 800x800 93 and 48, 262k on 384x384 128 and 67,
+// 1M on 640x640 320 and 173.  Records loaded two batches ahead measured
+// 5-10% slower; a workgroup of four waves on a quadrant, each evaluating a
+// quarter of the entries and all blending one channel each, 309 at the last.
+struct BlockLds {
+  float4 a[64 + 4];      // x, y, conic a, 2 b
+  float4 b[64 + 4];      // conic c, opacity, candidate bound, 1-based list position
+  float channel[4][64 + 8];  // r, g, b, depth (rows 8 floats past a multiple of 64: other banks)
+};
+
+template <int kFrom>
+__device__ __forceinline__ float quad_lane(float v) {  // lane kFrom of the lane's quad
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kFrom * 0x55, 0xF, 0xF, true));
+}
+
+template <bool kDepth>
+__device__ __forceinline__ void render_fwd_block(const RenderFwdParams& p, BlockLds& s, int lane, int tile, int sub) {
+  const int g = lane & 3, pixel = lane >> 2;
+  const int sx0 = (tile % p.grid_x) * kBlockX + (sub & 3) * 4;
+  const int sy0 = (tile / p.grid_x) * kBlockY + (sub >> 2) * 4;
+  const int px = sx0 + (pixel & 3), py = sy0 + (pixel >> 2);
+  const bool in_image = px < p.W && py < p.H;
+  const float pfx = (float)px, pfy = (float)py;
+  const float rx0 = (float)sx0, rx1 = (float)(sx0 + 3), ry0 = (float)sy0, ry1 = (float)(sy0 + 3);
+  int2 rg = p.ranges[tile];
+  rg.x = imax(0, imin(rg.x, p.num_rendered));
+  rg.y = imax(rg.x, imin(rg.y, p.num_rendered));
+  const int n = rg.y - rg.x;
+  const int* const list = p.point_list + rg.x;
+
+  uint64_t live = __ballot(in_image);  // the four lanes of a pixel agree
+  float T = 1.0f, sum = 0.0f, weights = 0.0f;
+  int last = 0;  // of the records this lane evaluated
+
+  // loads ahead as in render_fwd_tile
+  int id_ahead = 0;
+  RecordRegs next;
+  next.r0 = next.r1 = next.r2 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (n > 0) {
+    next = load_record(p.records, checked_point(batch_entry(list, 0, imin(64, n), n, lane), p.num_points));
+    id_ahead = batch_entry(list, 64, imin(64, n - 64), n, lane);
+  }
+  for (int base = 0; base < n; base += 64) {
+    if (live == 0) break;
+    const int cnt = imin(64, n - base);
+    const bool signed_zero = __ballot(lane < cnt && !(next.r0.z > 0.0f)) != 0;  // as in render_fwd_tile
+    const uint64_t todo = __ballot(lane < cnt && extents_meet(next.r0.x, next.r0.y, __float_as_uint(next.r2.w), rx0,
+                                                              rx1, ry0, ry1));
+    const int count = __popcll(todo);
+    if ((todo >> lane) & 1) {
+      const int at = __popcll(todo & ((1ull << lane) - 1));
+      s.a[at] = make_float4(next.r0.x, next.r0.y, next.r0.z, 2.0f * next.r0.w);
+      s.b[at] = make_float4(next.r1.x, next.r1.y, __uint_as_float(cand_threshold(next.r1.w)),
+                            __int_as_float(base + lane + 1));
+      s.channel[0][at] = next.r2.x;
+      s.channel[1][at] = next.r2.y;
+      s.channel[2][at] = next.r2.z;
+      s.channel[3][at] = next.r1.z;
+    }
+    if (lane < 4) {  // fills the last step: opacity 0 blends nowhere
+      s.a[count + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      s.b[count + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s.channel[c][count + lane] = 0.0f;
+    }
+    next = load_record(p.records, checked_point(id_ahead, p.num_points));
+    id_ahead = batch_entry(list, base + 128, imin(64, n - base - 128), n, lane);
+    auto step = [&](const float4& a, const float4& b, int i) {
+      const float4 f = *reinterpret_cast<const float4*>(&s.channel[g][i]);
+      const float dx = a.x - pfx;
+      const float dy = a.y - pfy;
+      const float q = conic_q_px(a.z * dx * dx, a.w * dx, b.x, dy);
+      uint64_t cand = live & __builtin_amdgcn_uicmp(__float_as_uint(q), __float_as_uint(b.z), kCmpULT);
+      if (signed_zero) cand |= live & __builtin_amdgcn_fcmpf(q, 0.0f, kCmpOEQ);
+      if (cand == 0) return;
+      const float alpha = fminf(kAlphaMax, b.y * exp_sw_q(q));
+      uint64_t ok = cand & __builtin_amdgcn_fcmpf(alpha, kAlphaMin, kCmpOGE);
+      // a record that does not blend has alpha 0: T stays and the sums add an exact 0
+      const float own = __builtin_amdgcn_inverse_ballot_w64(ok) ? alpha : 0.0f;
+      float x0 = quad_lane<0>(own), x1 = quad_lane<1>(own), x2 = quad_lane<2>(own), x3 = quad_lane<3>(own);
+      float t1 = T * (1.0f - x0), t2 = t1 * (1.0f - x1), t3 = t2 * (1.0f - x2), t4 = t3 * (1.0f - x3);
+      // T never grows and a live pixel's is at least 1e-4, so a pixel stops in this step when
+      // it ends below that: at its first such record, which it does not blend
+      const uint64_t fin = live & __builtin_amdgcn_fcmpf(t4, kTransmittanceMin, kCmpOLT);
+      if (fin != 0) {
+        const bool stops = __builtin_amdgcn_inverse_ballot_w64(fin);
+        const int at = !stops ? 4 : t1 < kTransmittanceMin ? 0 : t2 < kTransmittanceMin ? 1 :
+                       t3 < kTransmittanceMin ? 2 : 3;
+        if (at <= 0) { x0 = 0.0f; t1 = T; }
+        if (at <= 1) { x1 = 0.0f; t2 = t1; }
+        if (at <= 2) { x2 = 0.0f; t3 = t2; }
+        if (at <= 3) { x3 = 0.0f; t4 = t3; }
+        ok &= __ballot(g < at);
+        live &= ~fin;
+      }
+      const float c0 = x0 * T, c1 = x1 * t1, c2 = x2 * t2, c3 = x3 * t3;
+      if (kDepth || g < 3) {
+        sum = fmaf(f.x, c0, sum);
+        sum = fmaf(f.y, c1, sum);
+        sum = fmaf(f.z, c2, sum);
+        sum = fmaf(f.w, c3, sum);
+      }
+      weights = weights + c0;
+      weights = weights + c1;
+      weights = weights + c2;
+      weights = weights + c3;
+      last = __builtin_amdgcn_inverse_ballot_w64(ok) ? __float_as_int(b.w) : last;
+      T = t4;
+    };
+    // two steps a turn, each with the other's records read ahead of it (the fill past the end)
+    float4 a0 = s.a[g], b0 = s.b[g];
+    for (int i = 0; i < count; i += 8) {
+      const int i1 = imin(i + 4, count), i2 = imin(i + 8, count);
+      const float4 a1 = s.a[i1 + g], b1 = s.b[i1 + g];
+      step(a0, b0, i);
+      a0 = s.a[i2 + g];
+      b0 = s.b[i2 + g];
+      step(a1, b1, i1);
+    }
+  }
+  last = imax(last, __builtin_amdgcn_update_dpp(0, last, 0xB1, 0xF, 0xF, true));  // quad_perm [1,0,3,2]
+  last = imax(last, __builtin_amdgcn_update_dpp(0, last, 0x4E, 0xF, 0xF, true));  // quad_perm [2,3,0,1]
+  if (in_image) {
+    const int P = p.W * p.H, pix = py * p.W + px;
+    if (g < 3)
+      p.out_color[g * P + pix] = sum + T * p.bg[g];
+    else
+      p.out_depth[pix] = kDepth ? sum : 0.0f;
+    if (g == 0) p.n_contrib[pix] = last;
+    if (g == 1) p.out_alpha[pix] = weights;
+  }
+}
+
+template <bool kDepth>
+__global__ __launch_bounds__(64) void render_fwd_block_kernel(RenderFwdParams p) {
+  __shared__ BlockLds s;
+  const int lane = threadIdx.x;
+  const int unit = xcd_unit(blockIdx.x, p.num_tiles * 16);
+  if (unit < p.num_tiles * 16)  // else grid padding
+    render_fwd_block<kDepth>(p, s, lane, p.tile_order ? p.tile_order[unit >> 4] : unit >> 4, unit & 15);
+  clear_share(p, lane);
+}
+
+// Where the 4x4 blocks are faster than the quadrants (times in us, quadrants
+// and blocks): up to 1600 tiles (1M Gaussians on 640x480 151 and 138, 60k on
+// 487x273 34 and 18); up to 2600 with at most 1.25M pairs (300k on 800x800 92
+// and 73, 600k 137 and 123, 300k on 1000x500 74 and 71, but 1M on 960x640, 1.7M
+// pairs, 131 and 165) or with 4 to 12 pairs per Gaussian (500k mid-sized splats on
+// 700x700 198 and 117).  Above 12 pairs per Gaussian opaque pixels end the
+// walks early and the records' loads weigh more (640x480 37 and 47); above
+// 2600 tiles the quadrants fill the chip (300k on 1280x720 79 and 95).
+static bool blocks_pay(int64_t num_tiles, int64_t num_rendered, int64_t num_points) {
+  if (num_tiles > 2600 || num_rendered > 12 * num_points) return false;
+  return num_tiles <= 1600 || num_rendered <= 1250000 || num_rendered > 4 * num_points;
+}
+
 // The order in which the blend kernels take the tiles: longest list first,
 // by a counting sort over 256 classes of the list length (4 pairs wide
 // below 512, 64 wide above, the last class open; one workgroup).  The
@@ -465,6 +637,12 @@ static int launch_render_fwd(const RenderFwdParams& p, bool flow, hipStream_t s)
       launch_render_fwd_as<true, true, false>(p, grid, 0, s);
     else
       launch_render_fwd_as<true, false, false>(p, grid, 0, s);
+  } else if (blocks_pay(p.num_tiles, p.num_rendered, p.num_points)) {
+    const dim3 blocks(gs::xcd_grid(p.num_tiles * 16));
+    if (p.compute_depth)
+      hipLaunchKernelGGL((render_fwd_block_kernel<true>), blocks, dim3(64), 0, s, p);
+    else
+      hipLaunchKernelGGL((render_fwd_block_kernel<false>), blocks, dim3(64), 0, s, p);
   } else {
     if (p.compute_depth)
       launch_render_fwd_as<false, true, false>(p, grid, 0, s);
