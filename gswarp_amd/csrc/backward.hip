@@ -9,10 +9,10 @@
 // divided by max(1-alpha, 1e-5) per blended Gaussian, reverse recurrences for
 // colour, depth and alpha, the background term).  Per Gaussian each lane
 // sums its pixels' pixel moments and colour / depth terms; the wave reduces
-// them through LDS (a transposed store and per-column sums for one-column
-// slices, two lane-swap folds for the whole tile) into a per-wave slot, which
-// is reduced and sent to global memory with one float atomic per component
-// at the next Gaussian (skipped for a zero sum).
+// them (one-column slices: a transposed store to LDS, per-column sums and DPP
+// sums of the columns; the whole tile: two lane-swap folds into an LDS slot
+// that is reduced at the next Gaussian) and sends them to global memory with
+// one float atomic per component (skipped for a zero sum).
 // The blend decisions are exactly the forward's (exp_sw is evaluated only in
 // a thin band above the record's power cutoff where the decision needs it);
 // gradient values use the hardware exponential and reciprocal.
@@ -131,25 +131,27 @@ __device__ __forceinline__ void flush_slot(const float* slot, int gid, int lane,
 }
 
 // Column-slice reduction through LDS (kCols == 1: a lane's pixels lie in the
-// column lane % 8 and share its dx).  Cross-lane VALU moves are the slow
-// part of a wave-wide sum (a v_permlane swap costs four fast adds), so the
-// wave transposes its sums through LDS instead.  The seven per-lane sums
-// (v, v dy, v dy^2 and the three colour and the depth terms) are stored so
-// that the eight lanes of one column hold a contiguous group of 8 floats:
-// component c of lane l at float
+// column lane % 8 and share its dx).  A wave-wide sum by cross-lane VALU moves
+// alone is slow (a v_permlane swap costs four fast adds), so the wave
+// transposes its sums through LDS first.  The seven per-lane sums (v, v dy,
+// v dy^2 and the three colour and the depth terms) are stored so that the
+// eight lanes of one column hold a contiguous group of 8 floats: component c
+// of lane l at float
 //   c * 64 + col * 8 + ((row + 4 (col / 4)) % 8),   col = l % 8, row = l / 8
 // (the rotation by 4 (col / 4) puts each half-wave's 32 stores on 32 banks).
-// Lane 8 c + col (c < 7; lanes 56-63 repeat c = 6) reads its group as two
-// float4 and adds them: the column sum S of component c; with the column's
-// dx it forms S dx and S dx^2, the dx moments (used for c = 0 and 1).  These
-// go to the slot: S at float lane, S dx at 64 + lane, S dx^2 at 128 + lane.
-// The slot is reduced at the next Gaussian, or at the slice's end: lane
-// 2 k + h (k < 10) reads the float4 of columns 4 h .. 4 h + 3 of output k and
-// adds it, the lane pair adds its two sums (one DPP add) and the even lane
-// sends output k with one atomic.  Outputs 0-6 are the column sums (grad
-// components 5, 1, 4, 6, 7, 8, 9), 7 sum v dx (component 0), 8 sum v dy dx
-// (3) and 9 sum v dx^2 (2).
-constexpr int kColSlotFloats = 3 * 64;
+// Lane 8 c + col (c < 7; lanes 56-63 take c = 0 again) reads its group as two
+// float4 and adds them: the column sum S of component c, and with the
+// column's dx the dx moments, S dx in lanes 0-15 (c = 0, 1) and S dx^2 in
+// lanes 56-63.  The eight columns are then added by three DPP steps inside
+// each group of eight lanes (sum8_pair), and ten lanes send the ten outputs
+// with one atomic: lanes 8 c + 4 the sums (grad components 5, 1, 4, 6, 7, 8, 9),
+// lane 60 sum v dx^2 (2), lane 5 sum v dx (0) and lane 13 sum v dx dy (3).
+//
+// The kernel is bound by its LDS traffic about as much as by VALU issue (1M
+// Gaussians, 1080p: LDS active 1.52e8 of 2.4e8 CU cycles).  A second LDS stage
+// instead of the DPP steps (three stores a visit and a float4 read of them at
+// the next visit) issued 2.28e8 vector instructions to these 2.4e8, but left
+// the LDS active 1.52e8 cycles to these 1.15e8: fwd+bwd 941 us to 905.
 constexpr int kColRawFloats = 7 * 64;
 
 __device__ __forceinline__ int col_raw_offset(int lane) {
@@ -157,44 +159,37 @@ __device__ __forceinline__ int col_raw_offset(int lane) {
   return col * 8 + ((row + 4 * (col >> 2)) & 7);
 }
 
-// float4 index (in the raw area) of the half of its group that a lane reads
-// first; the other is this ^ 1.  Odd components start with the upper half:
-// 16 lanes (two components) are served at once, and their groups lie 64
-// floats apart, so with both components reading the same half every access
-// met two lanes on each of half the banks.  1M Gaussians, 1080p: LDS conflict
-// cycles 3.1e7 -> 0.6e7 of 1.8e8 active ones, fwd+bwd 963 -> 947 us.
+// float4 index of the half of its group that a lane reads first; the other is
+// this ^ 1.  Odd components start with the upper half: 16 lanes (two
+// components) are served at once, and their groups lie 64 floats apart, so
+// with both components reading the same half every access met two lanes on
+// each of half the banks.  1M Gaussians, 1080p: LDS conflict cycles 3.1e7 ->
+// 0.6e7 of 1.8e8 active ones, fwd+bwd 963 -> 947 us.
 __device__ __forceinline__ int col_group_index(int lane) {
-  return imin(lane >> 3, 6) * 16 + (lane & 7) * 2 + ((lane >> 3) & 1);
+  const int group = lane >> 3;
+  return (group == 7 ? 0 : group) * 16 + (lane & 7) * 2 + (group & 1);
 }
 
-// float4 index (in the slot) that lane 2 k + h reads for output k
-__device__ __forceinline__ int col_flush_index(int lane) {
-  const int k = lane >> 1, h = lane & 1;
-  if (k >= 10) return 0;
-  const int f = k < 7 ? 8 * k : (k == 7 ? 64 : (k == 8 ? 72 : 128));
-  return (f >> 2) + h;
+// grad component that a lane sends (-1: none), lanes 8 c + 4 from the nibbles of a constant
+__device__ __forceinline__ int col_component(int lane) {
+  if (lane == 5) return 0;
+  if (lane == 13) return 3;
+  return (lane & 7) != 4 ? -1 : (int)((0x29876415u >> (4 * (lane >> 3))) & 15);
 }
 
-// grad component that lane 2 k sends (-1: none), stored in the nibbles of a constant
-__device__ __forceinline__ int col_flush_component(int lane) {
-  if (lane >= 20 || (lane & 1)) return -1;
-  return (int)((0x2309876415ull >> (4 * (lane >> 1))) & 15);
-}
-
-__device__ __forceinline__ void flush_col_slot(float4 v, int gid, int comp, float* grad_gauss) {
-  float t = (v.x + v.y) + (v.z + v.w);
-  t = t + dpp_mov<0xB1, 0xF>(t);  // quad_perm [1,0,3,2]: the pair partner's sum
-  // The Gaussian's row is wave-uniform: its address is formed on the scalar
-  // unit, and each lane adds only its component's offset.
-  const uint64_t row = grad_row(grad_gauss, gid);
-  if (comp >= 0 && t != 0.0f) global_add(row, (unsigned)comp, t);
+// The sums of a and of b over each group of eight lanes: a's in lane 4 of the
+// group, b's in lane 5 (the other lanes hold partial sums).  The first step
+// exchanges, between the lanes of a pair, the value that the other one sums.
+__device__ __forceinline__ float sum8_pair(float a, float b, bool odd) {
+  float x = (odd ? b : a) + dpp_mov<0xB1, 0xF>(odd ? a : b);  // quad_perm [1,0,3,2]
+  x = x + dpp_mov<0x4E, 0xF>(x);                               // quad_perm [2,3,0,1]
+  return x + dpp_mov<0x114, 0xF>(x);                           // row_shr:4
 }
 
 // The wave's LDS besides the records: the fold slot of wave_fold10, or the
-// column slot and the transposed sums.
+// transposed sums.
 constexpr int kSlotLdsFloats =
-    (kSlotFloats + kSlotPad) > (kColSlotFloats + kColRawFloats) ? (kSlotFloats + kSlotPad)
-                                                                : (kColSlotFloats + kColRawFloats);
+    (kSlotFloats + kSlotPad) > kColRawFloats ? (kSlotFloats + kSlotPad) : kColRawFloats;
 
 // A record's pixel classes as thresholds on the bits of q: for q >= +0 (sign
 // bit clear) bits(q) < cand exactly when q <= qcut (a candidate) and
@@ -389,11 +384,10 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
   }
   if (max_lc <= lo) return;
   const int flush_comp = lane < kSlotFloats / 4 ? slot_component(lane >> 2) : -1;  // kCols == 2
-  float* const col_raw = s_slot + kColSlotFloats;  // kCols == 1: the column slot, then the sums
+  float* const col_raw = s_slot;  // kCols == 1
   const int raw_ofs = col_raw_offset(lane);
   const int raw_grp = col_group_index(lane);
-  const int col_fidx = col_flush_index(lane);
-  const int col_fcomp = col_flush_component(lane);
+  const int col_comp = col_component(lane);
   int slot_gid = -1;  // Gaussian whose sums the slot holds (wave-uniform), -1: none
 
   // Batches of 64 list entries, back to front: [bs, batch_end).  The loads
@@ -590,10 +584,7 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
         // and W/2, H/2 factors are per Gaussian and applied once, when the
         // per-Gaussian backward turns the sums into 2D gradients.
         if constexpr (kCols == 1) {
-          // The transposed store of this Gaussian's sums, then (the wave's LDS
-          // operations complete in order) the reads of the previous Gaussian's
-          // slot and of this Gaussian's column groups, and the new slot after
-          // the flush.
+          // the wave's LDS operations complete in order
           col_raw[raw_ofs] = sv[0];
           col_raw[64 + raw_ofs] = svy[0];
           col_raw[128 + raw_ofs] = svyy;
@@ -601,16 +592,13 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
           col_raw[256 + raw_ofs] = sg;
           col_raw[320 + raw_ofs] = sb;
           col_raw[384 + raw_ofs] = sd;
-          const float4 prev = reinterpret_cast<const float4*>(s_slot)[col_fidx];
           const float4 ga = reinterpret_cast<const float4*>(col_raw)[raw_grp];
           const float4 gb = reinterpret_cast<const float4*>(col_raw)[raw_grp ^ 1];
-          if (slot_gid >= 0) flush_col_slot(prev, slot_gid, col_fcomp, p.grad_gauss);
-          slot_gid = __builtin_amdgcn_readlane(batch_id, jj);
+          const uint64_t row = grad_row(p.grad_gauss, __builtin_amdgcn_readlane(batch_id, jj));
           const float col_sum = ((ga.x + ga.y) + (ga.z + ga.w)) + ((gb.x + gb.y) + (gb.z + gb.w));
           const float col_dx = col_sum * dx[0];
-          s_slot[lane] = col_sum;
-          s_slot[64 + lane] = col_dx;
-          s_slot[128 + lane] = col_dx * dx[0];
+          const float out = sum8_pair(lane < 56 ? col_sum : col_dx * dx[0], col_dx, lane & 1);
+          if (col_comp >= 0 && out != 0.0f) global_add(row, (unsigned)col_comp, out);
         } else {
           float m[3];
           float g[kGradFloats];
@@ -655,12 +643,7 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
     for (int k = 0; k < kPix; ++k) seg.map_out[64 * k + lane] = make_float2(Ti[k], S[k]);
     return;
   }
-  if (slot_gid >= 0) {
-    if constexpr (kCols == 1)
-      flush_col_slot(reinterpret_cast<const float4*>(s_slot)[col_fidx], slot_gid, col_fcomp, p.grad_gauss);
-    else
-      flush_slot(s_slot, slot_gid, lane, flush_comp, p.grad_gauss);
-  }
+  if (kCols > 1 && slot_gid >= 0) flush_slot(s_slot, slot_gid, lane, flush_comp, p.grad_gauss);
 }
 
 // How a tile is split over waves.  With small Gaussians (a few tiles each)
@@ -814,7 +797,7 @@ template <bool kDepth, int kPix>
 __global__ __launch_bounds__(64, 6) void render_bwd_segments_kernel(RenderBwdParams p, const int* __restrict__ walk,
                                                                     float2* __restrict__ maps, int max_segments) {
   __shared__ float4 s_rec[3 * 64];
-  __shared__ __align__(16) float s_slot[kColSlotFloats + kColRawFloats];
+  __shared__ __align__(16) float s_slot[kColRawFloats];
   render_bwd_segment<kDepth, kPix, false>(p, walk, maps, max_segments, s_rec, s_slot);
 }
 
