@@ -406,8 +406,8 @@ __global__ __launch_bounds__(64) void render_fwd_kernel(RenderFwdParams p) {
 // 5-10% slower; a workgroup of four waves on a quadrant, each evaluating a
 // quarter of the entries and all blending one channel each, 309 at the last.
 struct BlockLds {
-  float4 a[64 + 4];      // x, y, conic a, 2 b
-  float4 b[64 + 4];      // conic c, opacity, candidate bound, 1-based list position
+  float4 a[64 + 8];      // x, y, conic a, 2 b
+  float4 b[64 + 8];      // conic c, opacity, candidate bound, 1-based list position
   float channel[4][64 + 8];  // r, g, b, depth (rows 8 floats past a multiple of 64: other banks)
 };
 
@@ -450,6 +450,10 @@ __device__ __forceinline__ void render_fwd_block(const RenderFwdParams& p, Block
     const uint64_t todo = __ballot(lane < cnt && extents_meet(next.r0.x, next.r0.y, __float_as_uint(next.r2.w), rx0,
                                                               rx1, ry0, ry1));
     const int count = __popcll(todo);
+    // A record's colour or depth that is not finite stays with the pixels that
+    // blend it: its product with an alpha of 0 would not be 0 elsewhere.
+    const float channels = (next.r2.x + next.r2.y) + (next.r2.z + next.r1.z);
+    const bool non_finite = (__ballot(!(fabsf(channels) < INFINITY)) & todo) != 0;
     if ((todo >> lane) & 1) {
       const int at = __popcll(todo & ((1ull << lane) - 1));
       s.a[at] = make_float4(next.r0.x, next.r0.y, next.r0.z, 2.0f * next.r0.w);
@@ -460,7 +464,7 @@ __device__ __forceinline__ void render_fwd_block(const RenderFwdParams& p, Block
       s.channel[2][at] = next.r2.z;
       s.channel[3][at] = next.r1.z;
     }
-    if (lane < 4) {  // fills the last step: opacity 0 blends nowhere
+    if (lane < 8) {  // fills the last two steps: opacity 0 blends nowhere
       s.a[count + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       s.b[count + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
@@ -469,7 +473,7 @@ __device__ __forceinline__ void render_fwd_block(const RenderFwdParams& p, Block
     next = load_record(p.records, checked_point(id_ahead, p.num_points));
     id_ahead = batch_entry(list, base + 128, imin(64, n - base - 128), n, lane);
     auto step = [&](const float4& a, const float4& b, int i) {
-      const float4 f = *reinterpret_cast<const float4*>(&s.channel[g][i]);
+      float4 f = *reinterpret_cast<const float4*>(&s.channel[g][i]);
       const float dx = a.x - pfx;
       const float dy = a.y - pfy;
       const float q = conic_q_px(a.z * dx * dx, a.w * dx, b.x, dy);
@@ -496,6 +500,12 @@ __device__ __forceinline__ void render_fwd_block(const RenderFwdParams& p, Block
         ok &= __ballot(g < at);
         live &= ~fin;
       }
+      if (non_finite) {
+        f.x = x0 != 0.0f ? f.x : 0.0f;
+        f.y = x1 != 0.0f ? f.y : 0.0f;
+        f.z = x2 != 0.0f ? f.z : 0.0f;
+        f.w = x3 != 0.0f ? f.w : 0.0f;
+      }
       const float c0 = x0 * T, c1 = x1 * t1, c2 = x2 * t2, c3 = x3 * t3;
       if (kDepth || g < 3) {
         sum = fmaf(f.x, c0, sum);
@@ -511,9 +521,10 @@ __device__ __forceinline__ void render_fwd_block(const RenderFwdParams& p, Block
       T = t4;
     };
     // two steps a turn, each with the other's records read ahead of it (the fill past the end)
+    const int end = (count + 3) & ~3;
     float4 a0 = s.a[g], b0 = s.b[g];
-    for (int i = 0; i < count; i += 8) {
-      const int i1 = imin(i + 4, count), i2 = imin(i + 8, count);
+    for (int i = 0; i < end; i += 8) {
+      const int i1 = imin(i + 4, end), i2 = imin(i + 8, end);
       const float4 a1 = s.a[i1 + g], b1 = s.b[i1 + g];
       step(a0, b0, i);
       a0 = s.a[i2 + g];

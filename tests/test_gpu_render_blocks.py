@@ -4,11 +4,12 @@ opaque piles whose pixels stop at every position of a step."""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
 from gswarp_amd import configs
-from helpers import options
+from helpers import gpu_forward, options, oracle_forward, to_np
 from test_gpu_parity import _check_forward
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +43,17 @@ def test_block_edges_match_oracle(width, height, device):
     scene = _pile(200, width, height, (0.05, 0.9), device)
     _check_forward(scene, options())
     _check_forward(scene, options(compute_depth=False))
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_non_finite_colour_stays_with_its_pixels(value, device):
+    """A step evaluates four records at a pixel; one that the pixel does not blend adds nothing, whatever its colour."""
+    scene = _pile(131, 37, 29, (0.05, 0.5), device)
+    scene["colors_precomp"] = torch.rand(131, 3, generator=torch.Generator().manual_seed(5)).to(device)
+    scene["colors_precomp"][::40] = value
+    got = to_np(gpu_forward(scene, options(), colors=True)["res"].color)
+    expected = oracle_forward(scene, compute_depth=True, colors=True)[1]["fwd"]["color"]
+    finite = np.isfinite(expected)
+    assert 0 < finite.sum() < finite.size
+    assert np.array_equal(np.isfinite(got), finite)
+    assert np.array_equal(got[finite], expected[finite])
