@@ -971,10 +971,11 @@ extern "C" int gs_bin_buckets(int32_t P, int32_t num_valid, int64_t num_entries,
   const int key_bits = gs_bit_length((long long)(depth_max - depth_min) + 1);
   hipLaunchKernelGGL(gs::bucket_depth_keys_kernel, dim3((P + 255) / 256), dim3(256), 0, s, P, cw, depths, depth_min,
                      keys, vals);
-  st = gs_sort_pairs_u32(P, 0, key_bits, keys, vals, keys_alt, vals_alt, ws + L.off_sort,
-                         L.off_cw - L.off_sort, stream);
+  int passes = 0;
+  st = gs_sort_pairs_u32_any(P, key_bits, keys, vals, keys_alt, vals_alt, ws + L.off_sort, L.off_cw - L.off_sort,
+                             &passes, stream);
   if (st != GS_OK) return st;
-  const int* order = gs_sort_num_passes(key_bits) % 2 ? vals_alt : vals;
+  const int* order = passes % 2 ? vals_alt : vals;
   const int first = P - V;
   mark(1);
 

@@ -25,7 +25,9 @@ static inline int gs_bit_length(long long v) {
 // order the caller may already have written into tile_order (order_ready,
 // gs_tile_order over the same ranges); gs_sort_tile_segments_ordered is
 // gs_sort_tile_segments whose workgroups take the tiles in the given order
-// (a permutation of the tiles, longest list first; null: tile order).
+// (a permutation of the tiles, longest list first; null: tile order);
+// gs_sort_pairs_u32_any is gs_sort_pairs_u32 on the low key_bits bits in
+// however many passes are fastest, reported in *passes.
 int gs_render_fwd_clear_ordered(int32_t image_width, int32_t image_height, int32_t num_points, int64_t num_rendered,
                                 const int32_t* ranges, const int32_t* point_list, const float* records,
                                 const float* background, int32_t compute_depth, float* out_color, float* out_depth,
@@ -34,3 +36,5 @@ int gs_render_fwd_clear_ordered(int32_t image_width, int32_t image_height, int32
 int gs_sort_tile_segments_ordered(int64_t n, uint64_t* keys, uint64_t* keys_alt, int32_t num_tiles,
                                   const int32_t* ranges, int32_t lo_bit, int32_t key_bits, int32_t value_bits,
                                   int32_t* point_list, int32_t write_keys, const int32_t* order, void* stream);
+int gs_sort_pairs_u32_any(int64_t n, int32_t key_bits, uint32_t* keys, int32_t* values, uint32_t* keys_alt,
+                          int32_t* values_alt, void* scratch, size_t scratch_bytes, int* passes, void* stream);

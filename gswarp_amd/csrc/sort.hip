@@ -1,40 +1,33 @@
 // Stable LSD radix sort of uint32 or uint64 keys (optionally with int32
 // values) for gfx950, on a bit field [lo_bit, lo_bit + key_bits) of the key.
 //
-// Per digit pass (reduce-then-scan; digits of at most 8 bits, the field split
-// evenly over ceil(bits / 8) passes):
-//   1. upsweep:   each 4096-element block counts its digits -> hist[digit][block].
+// Per digit pass (reduce-then-scan; digits of at most 8 bits, or 9 (Plan), the
+// field split evenly over ceil(bits / 8) passes):
+//   1. upsweep:   each block of 2048 to 8192 elements (Plan) counts its digits -> hist[digit][block].
 //   2. rowscan:   one workgroup per digit scans hist[digit][*] across blocks
 //                 (exclusive) and records the digit total.
 //   3. downsweep: each block ranks its elements stably, stages them in LDS in
 //                 digit order, and writes them out so that consecutive lanes
 //                 store consecutive addresses within each digit run.
-// The downsweep ranks with ballot matching: 8 ballots give each lane the set
+// The downsweep ranks with ballot matching: a ballot per digit bit gives each lane the set
 // of lanes holding its digit, the lane's rank among them is a popcount, and
 // only the lowest such lane updates the wave's counter, so ranks are stable
 // and keys whose digits take few values (the exponent bits of depths, the
 // high bits of tile ids) cause no LDS serialisation.
-// Element e of block b is handled by wave w = (e / 1024), item slot
-// i = (e % 1024) / 64, lane = e % 64, so processing slots in order with a
+// With k items a thread, element e of a block is handled by wave e / (64 k),
+// item slot (e % (64 k)) / 64 and lane e % 64, so processing slots in order with a
 // per-wave running counter preserves the input order among equal digits.
 #include "gs_capi.h"
+#include <initializer_list>
 
 namespace gs_sort {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-// Keys per thread of the radix passes: 16 (4096 per workgroup), or 32 for
-// sorts of at least kLargeSortKeys keys whose workgroup tile fits in 64 KB of
-// LDS, where the longer per-digit runs of each workgroup's scatter outweigh
-// the lower occupancy (and the halved number of histogram columns shortens
-// the digit-row scans).
-constexpr int kItems = 16;
-constexpr int kItemsLarge = 32;
-constexpr long long kLargeSortKeys = 1ll << 24;
-constexpr int kRadix = 256;
 
 typedef unsigned long long u64;
 
+template <int kWaveCount = kWaves>
 __device__ __forceinline__ unsigned block_exclusive_scan_u32(unsigned v, unsigned* lds_w, unsigned* total) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -48,7 +41,7 @@ __device__ __forceinline__ unsigned block_exclusive_scan_u32(unsigned v, unsigne
   __syncthreads();
   unsigned wave_off = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
+  for (int w = 0; w < kWaveCount; ++w) {
     const unsigned s = lds_w[w];
     if (w < wave) wave_off += s;
     tot += s;
@@ -66,7 +59,7 @@ __device__ __forceinline__ unsigned digit_of(K key, int shift, unsigned dmask) {
 }
 
 // Digit width of pass `pass` of `passes`: the key_bits are split as evenly as
-// possible (13 bits: 7 + 6, 26: 7 + 7 + 6 + 6), never above 8.  Narrow
+// possible (13 bits: 7 + 6, 26: 7 + 7 + 6 + 6).  Narrow
 // digits mean fewer destination runs per block in the scatter, and the
 // passes with wide digits are the ones whose writes scatter the most.
 static inline int pass_digit_bits(int key_bits, int passes, int pass) {
@@ -78,11 +71,13 @@ static inline int pass_digit_bits(int key_bits, int passes, int pass) {
 // of that bit, and the lanes agreeing with this lane's bit are ~(m ^ s).  The
 // update peers &= ~(m ^ s) is one v_bitop3_b32 per 32-bit half with truth
 // table 0x84 = S1 & ~(S0 ^ S2) (peers as S1; symmetric in S0 and S2).
-__device__ __forceinline__ u64 match_digit(unsigned d, bool valid) {
+template <int kBits>
+__device__ __forceinline__ u64 match_digit(unsigned d, bool valid, unsigned dmask) {
   const u64 v = __ballot(valid);
   unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
 #pragma unroll
-  for (int b = 0; b < 8; ++b) {
+  for (int b = 0; b < kBits; ++b) {
+    if (b >= 6 && !(dmask >> b)) break;  // uniform; a field splits into digits of mostly 6 bits or more
     const unsigned s = (unsigned)__builtin_amdgcn_sbfe((int)d, b, 1);
     const u64 m = __ballot(s != 0u);
     lo = __builtin_amdgcn_bitop3_b32((unsigned)m, lo, s, 0x84);
@@ -97,16 +92,18 @@ __device__ __forceinline__ u64 match_digit(unsigned d, bool valid) {
 // copies fall in different banks and a wave whose lanes share one digit
 // serialises 64 / kCopies deep instead of 64.
 constexpr int kCopies = 8;
-constexpr int kCopyStride = kRadix + 1;
 
-template <typename K, int kIt>
-__global__ __launch_bounds__(kThreads) void upsweep_kernel(const K* __restrict__ keys, long long n, int shift,
+template <typename K, int kThr, int kIt, int kBits>
+__global__ __launch_bounds__(kThr) void upsweep_kernel(const K* __restrict__ keys, long long n, int shift,
                                                           unsigned dmask, int nb, unsigned* __restrict__ hist) {
-  constexpr int kTile = kThreads * kIt;
+  constexpr int kTile = kThr * kIt;
+  constexpr int kRadix = 1 << kBits;
+  constexpr int kCopyStride = kRadix + 1;
+  static_assert(kThr >= kRadix, "a thread per digit");
   __shared__ unsigned h[kCopies * kCopyStride];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < kCopies * kCopyStride; i += kThreads) h[i] = 0;
+  for (int i = threadIdx.x; i < kCopies * kCopyStride; i += kThr) h[i] = 0;
   const long long base = (long long)blockIdx.x * kTile + wave * (64 * kIt) + lane;
   K key[kIt];
 #pragma unroll
@@ -121,6 +118,7 @@ __global__ __launch_bounds__(kThreads) void upsweep_kernel(const K* __restrict__
     if (base + i * 64 < n) atomicAdd(mine + digit_of(key[i], shift, dmask), 1u);
   __syncthreads();
   const int d = threadIdx.x;
+  if (kThr > kRadix && d >= kRadix) return;
   unsigned c = 0;
 #pragma unroll
   for (int k = 0; k < kCopies; ++k) c += h[k * kCopyStride + d];
@@ -168,20 +166,23 @@ __global__ __launch_bounds__(kThreads) void rowscan_kernel(int nb, unsigned* __r
   if (threadIdx.x == 0) digit_totals[blockIdx.x] = carry;
 }
 
-template <typename K, bool kValues, int kIt>
-__global__ __launch_bounds__(kThreads) void downsweep_kernel(const K* __restrict__ keys_in,
+template <typename K, bool kValues, int kThr, int kIt, int kBits>
+__global__ __launch_bounds__(kThr) void downsweep_kernel(const K* __restrict__ keys_in,
                                                             const int* __restrict__ vals_in,
                                                             K* __restrict__ keys_out, int* __restrict__ vals_out,
                                                             long long n, int shift, unsigned dmask, int nb,
                                                             const unsigned* __restrict__ hist,
                                                             const unsigned* __restrict__ digit_totals) {
-  constexpr int kTile = kThreads * kIt;
+  constexpr int kTile = kThr * kIt;
+  constexpr int kRadix = 1 << kBits;
+  static_assert(kThr >= kRadix, "a thread per digit");
+  constexpr int kW = kThr / 64;
   __shared__ K s_keys[kTile];
   __shared__ int s_vals[kValues ? kTile : 1];
-  __shared__ unsigned s_wcount[kWaves][kRadix];
+  __shared__ unsigned s_wcount[kW][kRadix];
   __shared__ unsigned s_dstart[kRadix];
   __shared__ long long s_gbase[kRadix];
-  __shared__ unsigned s_lds_w[kWaves];
+  __shared__ unsigned s_lds_w[kW];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -190,7 +191,7 @@ __global__ __launch_bounds__(kThreads) void downsweep_kernel(const K* __restrict
   const int block_count = (int)((n - block_base) < kTile ? (n - block_base) : kTile);
 
 #pragma unroll
-  for (int i = threadIdx.x; i < kWaves * kRadix; i += kThreads) (&s_wcount[0][0])[i] = 0;
+  for (int i = threadIdx.x; i < kW * kRadix; i += kThr) (&s_wcount[0][0])[i] = 0;
 
   K key[kIt];
   int val[kIt];
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(kThreads) void downsweep_kernel(const K* __restrict
   for (int i = 0; i < kIt; ++i) {
     const bool valid = (wave_base + i * 64) < n;
     const unsigned d = digit_of(key[i], shift, dmask);
-    const u64 peers = match_digit(d, valid);
+    const u64 peers = match_digit<kBits>(d, valid, dmask);
     unsigned before = 0;
     if (valid) before = s_wcount[wave][d];
     __builtin_amdgcn_wave_barrier();
@@ -224,21 +225,24 @@ __global__ __launch_bounds__(kThreads) void downsweep_kernel(const K* __restrict
   // the global base such that global position = s_gbase[d] + local position.
   {
     const int d = threadIdx.x;
+    const bool mine = kThr == kRadix || d < kRadix;
     unsigned run = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const unsigned c = s_wcount[w][d];
-      s_wcount[w][d] = run;
+    for (int w = 0; w < kW; ++w) {
+      const unsigned c = mine ? s_wcount[w][d] : 0u;
+      if (mine) s_wcount[w][d] = run;
       run += c;
     }
     unsigned tot;
-    const unsigned dstart = block_exclusive_scan_u32(run, s_lds_w, &tot);
+    const unsigned dstart = block_exclusive_scan_u32<kW>(run, s_lds_w, &tot);
     // digits above dmask do not occur in this pass (no table rows exist)
     const bool used = (unsigned)d <= dmask;
     unsigned gtot;
-    const unsigned gstart = block_exclusive_scan_u32(used ? digit_totals[d] : 0u, s_lds_w, &gtot);
-    s_dstart[d] = dstart;
-    s_gbase[d] = (long long)gstart + (long long)(used ? hist[(size_t)d * nb + blockIdx.x] : 0u) - (long long)dstart;
+    const unsigned gstart = block_exclusive_scan_u32<kW>(used ? digit_totals[d] : 0u, s_lds_w, &gtot);
+    if (mine) {
+      s_dstart[d] = dstart;
+      s_gbase[d] = (long long)gstart + (long long)(used ? hist[(size_t)d * nb + blockIdx.x] : 0u) - (long long)dstart;
+    }
   }
   __syncthreads();
 
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(kThreads) void downsweep_kernel(const K* __restrict
 
 #pragma unroll
   for (int j = 0; j < kIt; ++j) {
-    const int p = j * kThreads + threadIdx.x;
+    const int p = j * kThr + threadIdx.x;
     if (p < block_count) {
       const K k = s_keys[p];
       const long long gp = s_gbase[digit_of(k, shift, dmask)] + p;
@@ -268,73 +272,123 @@ __global__ __launch_bounds__(kThreads) void downsweep_kernel(const K* __restrict
   }
 }
 
-static inline int items_for(long long n, size_t key_bytes, bool values) {
-  const size_t tile_bytes = (size_t)kThreads * kItemsLarge * (key_bytes + (values ? sizeof(int) : 0));
-  return (n >= kLargeSortKeys && tile_bytes <= 65536) ? kItemsLarge : kItems;
+// How a sort is split: threads and keys per thread of a workgroup, bits of the
+// widest digit.
+struct Plan {
+  int threads, items, digit_bits;
+  int tile() const { return threads * items; }
+  int64_t blocks(int64_t n) const { return (n + tile() - 1) / tile(); }
+  int passes(int key_bits) const { return (key_bits + digit_bits - 1) / digit_bits; }
+  // the histogram rows and the digit totals
+  size_t scratch_bytes(int64_t n) const { return ((size_t)blocks(n) + 1) * (sizeof(unsigned) << digit_bits); }
+};
+// What a pass takes for n keys (us, upsweep + rowscan + downsweep of u32 pairs
+// unless said otherwise):
+// - kDense, 4096 keys a workgroup: 36 at 5M (kMedium 36, 2048 keys and 512
+//   threads 50).  Below about 2M keys it leaves CUs without a workgroup and
+//   lasts as long as the sixteen ranking steps of a wave.
+// - kMedium, half the keys a thread: 19.8 at 1M (kDense 22.7); 2.9M u64 keys
+//   24.4 (24.5).
+// - kSmall, a quarter of the keys a thread: 13.1 at 500k (kMedium 14.1, kDense
+//   17.4); 440k u64 keys 13.5 (14.4, 17.1); but 20.3 at 1M (19.8).
+// - kWide, kSmall's split with digits of 9 bits: a pass costs 15.3 at 500k, and
+//   the 26 bits of ordinary depths take three passes instead of four: the whole
+//   sort 72 -> 48 (kDense to kWide).  At 5M the scatter's 512 runs cost
+//   more than the saved pass (2048, 4096 and 8192 keys a workgroup alike).
+// - kLarge: the longer runs of each workgroup's scatter outweigh the lower
+//   occupancy, where the tile fits in 64 KB of LDS.
+constexpr Plan kDense = {256, 16, 8};
+constexpr Plan kLarge = {256, 32, 8};
+constexpr Plan kMedium = {256, 8, 8};
+constexpr Plan kSmall = {512, 4, 8};
+constexpr Plan kWide = {512, 4, 9};
+constexpr int64_t kSmallKeys = 768 << 10, kMediumKeys = 2 << 20, kWideKeys = 3 << 19, kLargeKeys = 1 << 24;
+
+// The scratch that any plan of up to n keys needs (it never falls as n grows,
+// so that scratch made for a capacity serves every smaller sort).
+static inline size_t scratch_size(int64_t n) {
+  const auto upto = [n](const Plan& p, int64_t limit) { return p.scratch_bytes(n < limit ? n : limit); };
+  size_t bytes = kDense.scratch_bytes(n);
+  for (size_t b : {upto(kSmall, kSmallKeys), upto(kMedium, kMediumKeys), upto(kWide, kWideKeys)})
+    if (b > bytes) bytes = b;
+  return (bytes + 255) & ~(size_t)255;
 }
-static inline int num_blocks(long long n, int items = kItems) {
-  const long long tile = (long long)kThreads * items;
-  return (int)((n + tile - 1) / tile);
+
+// Scratch of kDense's size is always enough: a plan that needs more is passed
+// over when the caller's scratch is smaller.
+static inline Plan plan_for(int64_t n, int key_bits, size_t pair_bytes, size_t scratch_bytes, bool wide) {
+  const auto fits = [&](const Plan& p) { return p.scratch_bytes(n) <= scratch_bytes; };
+  if (wide && n <= kWideKeys && kWide.passes(key_bits) < kDense.passes(key_bits) && fits(kWide)) return kWide;
+  if (n <= kSmallKeys && fits(kSmall)) return kSmall;
+  if (n <= kMediumKeys && fits(kMedium)) return kMedium;
+  if (n >= kLargeKeys && kLarge.tile() * pair_bytes <= 65536) return kLarge;
+  return kDense;
 }
 
 template <typename K, bool kValues>
+struct Buffers {
+  K *keys, *keys_out;
+  int *vals, *vals_out;
+};
+
+template <int kThr, int kIt, int kBits, typename K, bool kValues>
+static void sort_pass(const Buffers<K, kValues>& b, int64_t n, int shift, unsigned dmask, unsigned* hist,
+                      unsigned* digit_totals, hipStream_t s) {
+  const int nb = (int)Plan{kThr, kIt, kBits}.blocks(n);
+  hipLaunchKernelGGL((upsweep_kernel<K, kThr, kIt, kBits>), dim3(nb), dim3(kThr), 0, s, b.keys, (long long)n, shift,
+                     dmask, nb, hist);
+  hipLaunchKernelGGL(rowscan_kernel, dim3(dmask + 1), dim3(kThreads), 0, s, nb, hist, digit_totals);
+  hipLaunchKernelGGL((downsweep_kernel<K, kValues, kThr, kIt, kBits>), dim3(nb), dim3(kThr), 0, s, b.keys, b.vals,
+                     b.keys_out, b.vals_out, (long long)n, shift, dmask, nb, hist, digit_totals);
+}
+
+// kAnyDigits: the number of passes need not be gs_sort_num_passes(key_bits)
+template <typename K, bool kValues, bool kAnyDigits = false>
 static int sort_impl(int64_t n, int32_t lo_bit, int32_t key_bits, K* kin, K* kout, int* vin, int* vout,
-                     void* scratch, size_t scratch_bytes, hipStream_t s);
+                     void* scratch, size_t scratch_bytes, hipStream_t s, int* passes_out = nullptr) {
+  if (n < 0 || lo_bit < 0 || key_bits < 0 || lo_bit + key_bits > (int)(8 * sizeof(K)))
+    return GS_ERR_INVALID_ARGUMENT;
+  if (n > 0x7fffffffLL) return GS_ERR_OVERFLOW;
+  if (passes_out) *passes_out = 0;
+  if (n == 0 || key_bits == 0) return GS_OK;
+  if (!kin || !kout || !scratch || (kValues && (!vin || !vout))) return GS_ERR_INVALID_ARGUMENT;
+  if (scratch_bytes < ((kDense.scratch_bytes(n) + 255) & ~(size_t)255)) return GS_ERR_SCRATCH_TOO_SMALL;
+  const Plan plan = plan_for(n, key_bits, sizeof(K) + (kValues ? sizeof(int) : 0), scratch_bytes, kAnyDigits);
+  unsigned* hist = reinterpret_cast<unsigned*>(scratch);
+  unsigned* digit_totals = hist + ((size_t)plan.blocks(n) << plan.digit_bits);
+  const int passes = plan.passes(key_bits);
+  if (passes_out) *passes_out = passes;
+  Buffers<K, kValues> b = {kin, kout, vin, vout};
+  int shift = lo_bit;
+  for (int pass = 0; pass < passes; ++pass) {
+    const int bits = pass_digit_bits(key_bits, passes, pass);
+    const unsigned dmask = (1u << bits) - 1u;
+    if (kAnyDigits && plan.digit_bits == kWide.digit_bits)
+      sort_pass<kWide.threads, kWide.items, kWide.digit_bits>(b, n, shift, dmask, hist, digit_totals, s);
+    else if (plan.threads == kSmall.threads)
+      sort_pass<kSmall.threads, kSmall.items, 8>(b, n, shift, dmask, hist, digit_totals, s);
+    else if (plan.items == kMedium.items)
+      sort_pass<kMedium.threads, kMedium.items, 8>(b, n, shift, dmask, hist, digit_totals, s);
+    else if (plan.items == kLarge.items)
+      sort_pass<kLarge.threads, kLarge.items, 8>(b, n, shift, dmask, hist, digit_totals, s);
+    else
+      sort_pass<kDense.threads, kDense.items, 8>(b, n, shift, dmask, hist, digit_totals, s);
+    shift += bits;
+    b = {b.keys_out, b.keys, b.vals_out, b.vals};
+  }
+  return gs_status_from_hip(hipGetLastError());
+}
 
 }  // namespace gs_sort
 
 extern "C" int gs_sort_num_passes(int32_t key_bits) { return gs_passes_for_bits(key_bits); }
 
-extern "C" size_t gs_sort_scratch_bytes(int64_t n) {
-  if (n <= 0) return 0;
-  const size_t nb = (size_t)gs_sort::num_blocks(n);
-  const size_t bytes = (nb * gs_sort::kRadix + gs_sort::kRadix) * sizeof(unsigned);
-  return (bytes + 255) & ~(size_t)255;
-}
+extern "C" size_t gs_sort_scratch_bytes(int64_t n) { return n <= 0 ? 0 : gs_sort::scratch_size(n); }
 
-template <typename K, bool kValues>
-static int gs_sort::sort_impl(int64_t n, int32_t lo_bit, int32_t key_bits, K* kin, K* kout, int* vin,
-                              int* vout, void* scratch, size_t scratch_bytes, hipStream_t s) {
-  if (n < 0 || lo_bit < 0 || key_bits < 0 || lo_bit + key_bits > (int)(8 * sizeof(K)))
-    return GS_ERR_INVALID_ARGUMENT;
-  if (n > 0x7fffffffLL) return GS_ERR_OVERFLOW;
-  if (n == 0 || key_bits == 0) return GS_OK;
-  if (!kin || !kout || !scratch || (kValues && (!vin || !vout))) return GS_ERR_INVALID_ARGUMENT;
-  if (scratch_bytes < gs_sort_scratch_bytes(n)) return GS_ERR_SCRATCH_TOO_SMALL;
-  // the scratch query counts 16-key tiles, the most histogram columns
-  const int items = items_for(n, sizeof(K), kValues);
-  const int nb = num_blocks(n, items);
-  unsigned* hist = reinterpret_cast<unsigned*>(scratch);
-  unsigned* digit_totals = hist + (size_t)nb * kRadix;
-  const int passes = gs_passes_for_bits(key_bits);
-  int shift = lo_bit;
-  for (int pass = 0; pass < passes; ++pass) {
-    const int bits = pass_digit_bits(key_bits, passes, pass);
-    const unsigned dmask = (1u << bits) - 1u;
-    if (items == kItemsLarge) {
-      hipLaunchKernelGGL((upsweep_kernel<K, kItemsLarge>), dim3(nb), dim3(kThreads), 0, s, kin, (long long)n, shift,
-                         dmask, nb, hist);
-    } else {
-      hipLaunchKernelGGL((upsweep_kernel<K, kItems>), dim3(nb), dim3(kThreads), 0, s, kin, (long long)n, shift,
-                         dmask, nb, hist);
-    }
-    hipLaunchKernelGGL(rowscan_kernel, dim3(dmask + 1), dim3(kThreads), 0, s, nb, hist, digit_totals);
-    if (items == kItemsLarge) {
-      hipLaunchKernelGGL((downsweep_kernel<K, kValues, kItemsLarge>), dim3(nb), dim3(kThreads), 0, s, kin, vin,
-                         kout, vout, (long long)n, shift, dmask, nb, hist, digit_totals);
-    } else {
-      hipLaunchKernelGGL((downsweep_kernel<K, kValues, kItems>), dim3(nb), dim3(kThreads), 0, s, kin, vin, kout,
-                         vout, (long long)n, shift, dmask, nb, hist, digit_totals);
-    }
-    shift += bits;
-    K* tk = kin;
-    kin = kout;
-    kout = tk;
-    int* tv = vin;
-    vin = vout;
-    vout = tv;
-  }
-  return gs_status_from_hip(hipGetLastError());
+int gs_sort_pairs_u32_any(int64_t n, int32_t key_bits, uint32_t* keys, int32_t* values, uint32_t* keys_alt,
+                          int32_t* values_alt, void* scratch, size_t scratch_bytes, int* passes, void* stream) {
+  return gs_sort::sort_impl<unsigned, true, true>(n, 0, key_bits, keys, keys_alt, values, values_alt, scratch,
+                                                  scratch_bytes, (hipStream_t)stream, passes);
 }
 
 extern "C" int gs_sort_pairs_u64(int64_t n, int32_t key_bits, uint64_t* keys, int32_t* values,
@@ -406,7 +460,7 @@ __device__ __forceinline__ void rank_slots(const u64 (&key)[kSlots], const bool 
     rank[i] = 0;
     if (i < nslots) {
       const unsigned d = gs_sort::digit_of(key[i], shift, dmask);
-      const u64 peers = gs_sort::match_digit(d, valid[i]);
+      const u64 peers = gs_sort::match_digit<8>(d, valid[i], dmask);
       unsigned before = 0;
       if (valid[i]) before = wc[d];
       __builtin_amdgcn_wave_barrier();
@@ -433,22 +487,6 @@ constexpr int kSmallSlots = 16;
 constexpr int kSmallCap = 64 * kSmallSlots;  // 1024 keys
 constexpr int kSmallDigitBits = 9;
 constexpr int kSmallRadix = 1 << kSmallDigitBits;
-
-// Lanes of the wave holding the same kBits-bit digit d (among valid lanes);
-// the same per-bit ballot filtering as gs_sort::match_digit.
-template <int kBits>
-__device__ __forceinline__ u64 match_bits(unsigned d, bool valid) {
-  const u64 v = __ballot(valid);
-  unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
-#pragma unroll
-  for (int b = 0; b < kBits; ++b) {
-    const unsigned sb = (unsigned)__builtin_amdgcn_sbfe((int)d, b, 1);
-    const u64 m = __ballot(sb != 0u);
-    lo = __builtin_amdgcn_bitop3_b32((unsigned)m, lo, sb, 0x84);
-    hi = __builtin_amdgcn_bitop3_b32((unsigned)(m >> 32), hi, sb, 0x84);
-  }
-  return ((u64)hi << 32) | lo;
-}
 
 // Inclusive prefix sum over the 64 lanes: Hillis-Steele within each row of
 // 16 lanes by DPP row shifts (lanes shifted in from outside the row read 0),
@@ -508,7 +546,7 @@ __device__ __forceinline__ void small_segment_sort(long long n, u64* __restrict_
       rank[i] = 0;
       if (i < nslots) {
         const unsigned d = (unsigned)(key[i] >> shift) & dmask;
-        const u64 peers = match_bits<kSmallDigitBits>(d, valid[i]);
+        const u64 peers = gs_sort::match_digit<kSmallDigitBits>(d, valid[i], dmask);
         unsigned before = 0;
         if (valid[i]) before = s_wc[d];
         __builtin_amdgcn_wave_barrier();
