@@ -159,6 +159,66 @@ __global__ __launch_bounds__(256) void bucket_transpose_kernel(const int* __rest
   }
 }
 
+// Level-1 counts of up to kColumnChunks chunks into running positions, in
+// place: hist[c * B + b] becomes the number of entries of super-tile b in the
+// chunks before c, and totals[b] its entries in all chunks (the ranking adds
+// the super-tile's list start, which bucket_table_kernel finds from the
+// totals).  A workgroup takes kColumns neighbouring super-tiles, thread t the
+// rows [r k, (r + 1) k) of column t % kColumns, r = t / kColumns, held in
+// registers between the scan's two sides.
+//
+// One launch instead of the four of the transposed scan (two transposes, two
+// scan passes), which are bound by launches and latency at these sizes: 500k
+// splats on 1280x720 (about 1.6k chunks, 60 super-tiles) 23 us in four launches, now
+// 4.8, and the view 353 -> 335; 1M on 640x640 (4.1k chunks, 25 super-tiles)
+// 20 us, now 9.8.  Beyond, a thread's rows no longer fit its registers, and a
+// workgroup's strided reads of whole columns grow with the chunks while the
+// transposed scan spreads over the chip.
+constexpr int kColumns = 4;
+constexpr int kColumnRows = 16;  // most rows of a thread
+constexpr int kColumnChunks = 1024 / kColumns * kColumnRows;
+
+__global__ __launch_bounds__(1024) void bucket_column_scan_kernel(int nchunks, int B, int* __restrict__ hist,
+                                                                 int* __restrict__ totals) {
+  __shared__ int s_tot[1024 / 64][kColumns];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int b = blockIdx.x * kColumns + (threadIdx.x & (kColumns - 1));
+  const int rows = (nchunks + 1024 / kColumns - 1) / (1024 / kColumns);
+  const int c0 = threadIdx.x / kColumns * rows;
+  int v[kColumnRows];
+  int sum = 0;
+#pragma unroll
+  for (int q = 0; q < kColumnRows; ++q) {
+    const bool ok = q < rows && c0 + q < nchunks && b < B;
+    v[q] = hist[ok ? (size_t)(c0 + q) * B + b : 0];
+    v[q] = ok ? v[q] : 0;
+  }
+#pragma unroll
+  for (int q = 0; q < kColumnRows; ++q) sum += v[q];
+  int incl = sum;
+#pragma unroll
+  for (int off = kColumns; off < 64; off <<= 1) {
+    const int n = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += n;
+  }
+  if (lane >= 64 - kColumns) s_tot[wave][lane & (kColumns - 1)] = incl;
+  __syncthreads();  // also: every count of these columns has been read
+  int run = incl - sum, all = 0;
+#pragma unroll
+  for (int w = 0; w < 1024 / 64; ++w) {
+    const int t = s_tot[w][threadIdx.x & (kColumns - 1)];
+    if (w < wave) run += t;
+    all += t;
+  }
+  if (b >= B) return;
+  if (threadIdx.x < kColumns) totals[b] = all;
+#pragma unroll
+  for (int q = 0; q < kColumnRows; ++q) {
+    if (q < rows && c0 + q < nchunks) hist[(size_t)(c0 + q) * B + b] = run;
+    run += v[q];
+  }
+}
+
 // The clipped extent of a cover word's rectangle in super-tile (sx, sy):
 // tiles [x0, x1) x [y0, y1); empty when x1 <= x0 or y1 <= y0.
 struct Clip {
@@ -281,7 +341,8 @@ __global__ __launch_bounds__(64) void bucket_scatter_kernel(int V, const int4* _
                                                            const int* __restrict__ idx_sorted,
                                                            const unsigned* __restrict__ band_store,
                                                            const float4* __restrict__ records,
-                                                           const int* __restrict__ pos_cm, int nchunks, int nsx,
+                                                           const int* __restrict__ pos_cm,
+                                                           const int* __restrict__ base, int nchunks, int nsx,
                                                            int B, int bucket_bits, long long E,
                                                            int* __restrict__ e_idx,
                                                            unsigned long long* __restrict__ e_mask) {
@@ -312,6 +373,13 @@ __global__ __launch_bounds__(64) void bucket_scatter_kernel(int V, const int4* _
       int v[kPosBatch];
 #pragma unroll
       for (int q = 0; q < kPosBatch; ++q) v[q] = pos_cm[(size_t)c * B + imin(b0 + q * 64 + lane, B - 1)];
+      if (base) {  // positions within each super-tile's list
+        int at[kPosBatch];
+#pragma unroll
+        for (int q = 0; q < kPosBatch; ++q) at[q] = base[imin(b0 + q * 64 + lane, B - 1)];
+#pragma unroll
+        for (int q = 0; q < kPosBatch; ++q) v[q] += at[q];
+      }
 #pragma unroll
       for (int q = 0; q < kPosBatch; ++q)
         if (b0 + q * 64 + lane < B) cnt[b0 + q * 64 + lane] = v[q];
@@ -444,14 +512,16 @@ __global__ __launch_bounds__(64) void bucket_scatter_kernel(int V, const int4* _
 }
 
 // Per super-tile: its entry list [list_start[s], list_start[s + 1]) from the
-// scanned level-1 counts, and its level-2 chunks [chunk_start[s],
+// scanned level-1 counts (kTotals: from every super-tile's total), and its
+// level-2 chunks [chunk_start[s],
 // chunk_start[s + 1]); chunk_start[B] is the number of level-2 chunks.  Each
 // chunk g < nc2_max gets chunk_info[g] = (s, first entry, end entry), or
 // (-1, 0, 0) past the last chunk, so that a chunk's wave finds its entries
 // with one load.  Every workgroup scans the super-tiles itself (at most
 // kMaxSuper, four per thread) and fills 256 chunks, each finding its
 // super-tile by binary search; workgroup 0 also writes the two tables.
-__global__ __launch_bounds__(256) void bucket_table_kernel(const int* __restrict__ hist_incl, int nchunks, int B,
+template <bool kTotals>
+__global__ __launch_bounds__(256) void bucket_table_kernel(const int* __restrict__ counts, int nchunks, int B,
                                                           int nc2_max, int* __restrict__ list_start,
                                                           int* __restrict__ chunk_start,
                                                           int4* __restrict__ chunk_info) {
@@ -463,8 +533,27 @@ __global__ __launch_bounds__(256) void bucket_table_kernel(const int* __restrict
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int s = k * 256 + threadIdx.x;
-    start[k] = s > 0 && s < B ? hist_incl[(size_t)s * nchunks - 1] : 0;
-    end[k] = s < B ? hist_incl[(size_t)(s + 1) * nchunks - 1] : 0;
+    start[k] = !kTotals && s > 0 && s < B ? counts[(size_t)s * nchunks - 1] : 0;
+    end[k] = s < B ? counts[kTotals ? s : (size_t)(s + 1) * nchunks - 1] : 0;
+  }
+  if constexpr (kTotals) {
+    int entries = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      if (k * 256 >= B) break;
+      const int incl = wave_inclusive_scan_i32(end[k]);
+      if (lane == 63) s_tot[wave] = incl;
+      __syncthreads();
+      int before = 0, all = 0;
+      for (int w = 0; w < 256 / 64; ++w) {
+        before += w < wave ? s_tot[w] : 0;
+        all += s_tot[w];
+      }
+      start[k] = entries + before + incl - end[k];
+      end[k] = entries + before + incl;
+      entries += all;
+      __syncthreads();
+    }
   }
   int carry = 0;
 #pragma unroll
@@ -983,27 +1072,38 @@ extern "C" int gs_bin_buckets(int32_t P, int32_t num_valid, int64_t num_entries,
   const int nh = L.B * L.nchunks;
   const size_t lds_b = (size_t)L.B * sizeof(int);
   const size_t lds_d = (size_t)(L.nsx + 1) * (L.nsy + 1) * sizeof(int);
-  // counts chunk-major (each chunk writes one contiguous row), transposed to
-  // super-tile-major for the scan, and the scanned positions transposed back
-  // so that each ranking chunk reads one contiguous row
+  // counts chunk-major (each chunk writes one contiguous row), turned into
+  // running positions per super-tile: in place up to kColumnChunks chunks,
+  // else transposed to super-tile-major for the scan, and the scanned
+  // positions transposed back so that each ranking chunk reads one row
   hipLaunchKernelGGL(gs::bucket_count_kernel, dim3(L.nchunks), dim3(64), lds_d, s, V, first, P, order, cw,
                      cw_sorted, idx_sorted, L.nsx, L.nsy, L.nchunks, pos_cm);
-  hipLaunchKernelGGL(gs::bucket_transpose_kernel, dim3((L.B + 63) / 64, (L.nchunks + 63) / 64), dim3(256), 0, s,
-                     pos_cm, L.nchunks, L.B, 0, hist);
-  st = gs_scan_tiles(nh, hist, nullptr, nullptr, nullptr, hist_incl, info, ws + L.off_scan,
-                     L.off_info - L.off_scan, stream);
-  if (st != GS_OK) return st;
-  hipLaunchKernelGGL(gs::bucket_transpose_kernel, dim3((L.nchunks + 63) / 64, (L.B + 63) / 64), dim3(256), 0, s,
-                     hist_incl, L.B, L.nchunks, 1, pos_cm);
+  const dim3 table_grid((L.nc2_max + 255) / 256);
+  const int* base = nullptr;
+  if (L.nchunks <= gs::kColumnChunks) {
+    base = list_start;
+    hipLaunchKernelGGL(gs::bucket_column_scan_kernel, dim3((L.B + gs::kColumns - 1) / gs::kColumns), dim3(1024), 0, s,
+                       L.nchunks, L.B, pos_cm, hist);
+    hipLaunchKernelGGL((gs::bucket_table_kernel<true>), table_grid, dim3(256), 0, s, hist, L.nchunks, L.B, L.nc2_max,
+                       list_start, chunk_start, chunk_info);
+  } else {
+    hipLaunchKernelGGL(gs::bucket_transpose_kernel, dim3((L.B + 63) / 64, (L.nchunks + 63) / 64), dim3(256), 0, s,
+                       pos_cm, L.nchunks, L.B, 0, hist);
+    st = gs_scan_tiles(nh, hist, nullptr, nullptr, nullptr, hist_incl, info, ws + L.off_scan,
+                       L.off_info - L.off_scan, stream);
+    if (st != GS_OK) return st;
+    hipLaunchKernelGGL(gs::bucket_transpose_kernel, dim3((L.nchunks + 63) / 64, (L.B + 63) / 64), dim3(256), 0, s,
+                       hist_incl, L.B, L.nchunks, 1, pos_cm);
+    hipLaunchKernelGGL((gs::bucket_table_kernel<false>), table_grid, dim3(256), 0, s, hist_incl, L.nchunks, L.B,
+                       L.nc2_max, list_start, chunk_start, chunk_info);
+  }
   const int bucket_bits = gs_bit_length((long long)L.B - 1);
   hipLaunchKernelGGL(gs::bucket_scatter_kernel, dim3(L.nchunks), dim3(64), lds_b, s, V, cw_sorted, idx_sorted,
                      reinterpret_cast<const unsigned*>(band_store), reinterpret_cast<const float4*>(records),
-                     pos_cm, L.nchunks, L.nsx, L.B, bucket_bits, E, e_idx, e_mask);
+                     pos_cm, base, L.nchunks, L.nsx, L.B, bucket_bits, E, e_idx, e_mask);
   mark(2);
 
   // 3. level 2: per-tile lists
-  hipLaunchKernelGGL(gs::bucket_table_kernel, dim3((L.nc2_max + 255) / 256), dim3(256), 0, s, hist_incl, L.nchunks,
-                     L.B, L.nc2_max, list_start, chunk_start, chunk_info);
   hipLaunchKernelGGL(gs::bucket_tile_count_kernel, dim3(L.nc2_max), dim3(64), 0, s, chunk_info, (int)E, e_mask, cnt2);
   hipLaunchKernelGGL(gs::bucket_tile_prefix_kernel, dim3(L.B), dim3(1024), 0, s, chunk_start, L.nsx, L.grid_x,
                      L.grid_y, L.nc2_max, cnt2, tile_count);

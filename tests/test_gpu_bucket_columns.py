@@ -1,0 +1,47 @@
+"""The bucketed binning's running positions: scanned in place up to 4096 chunks of 256 Gaussians,
+transposed beyond.  The lists must be those of the depth-then-tile sort bit for bit."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from gswarp_amd import _pipeline, configs
+from helpers import gpu_forward, options
+
+pytestmark = pytest.mark.gpu
+
+
+def _pile(count, width, height, device):
+    """`count` splats of a pixel or two, all of them in view."""
+    scene = configs.make_scene(1, count=count, width=width, height=height, device=device)
+    g = torch.Generator().manual_seed(count)
+    pixel = 4.0 * 2.0 * scene["tanfovx"] / width
+    means = torch.rand(count, 3, generator=g) * 2.0 - 1.0
+    means[:, 0] *= 0.4 * width * pixel
+    means[:, 1] *= 0.4 * height * pixel
+    means[:, 2] *= 0.2
+    scene["means3D"] = means.to(device)
+    scene["scales"] = (pixel * (0.5 + torch.rand(count, 3, generator=g))).to(device)
+    scene["opacities"] = torch.full((count, 1), 0.5, device=device)
+    return scene
+
+
+@pytest.mark.parametrize("count,width,height", [
+    (1, 16, 16), (256, 130, 20), (257, 130, 140), (65_536, 400, 300), (65_537, 400, 300),
+    (3000, 4080, 4080),                          # 32 x 32 super-tiles
+    (1_048_576, 300, 260), (1_048_832, 300, 260),  # 4096 chunks, and more
+])
+def test_lists_match_the_depth_tile_sort(count, width, height, device, monkeypatch):
+    scene = _pile(count, width, height, device)
+    monkeypatch.setattr(_pipeline, "DEPTH_TILE_MIN_PAIRS_PER_GAUSSIAN", 0)
+    monkeypatch.setattr(_pipeline, "BUCKET_SIZING", "always")
+    outs = {}
+    for flow in ("buckets", "depth_tile"):
+        monkeypatch.setattr(_pipeline, "HEAVY_DATAFLOW", flow)
+        print(f"[columns] N={count} {width}x{height} {flow}", flush=True)
+        outs[flow] = gpu_forward(scene, options())["bins"]
+    a, b = outs["buckets"], outs["depth_tile"]
+    assert a.num_rendered == b.num_rendered >= count
+    assert torch.equal(a.point_list, b.point_list)
+    assert torch.equal(a.ranges, b.ranges)
