@@ -1621,8 +1621,9 @@ static int bin_packed_impl(int32_t P, const int32_t* radii, const float* records
   if (num_rendered == 0)
     return tile_ranges_impl(0, nullptr, tile_shift, 0, num_tiles, ranges, nullptr, ranges_cleared, s);
   if (!workspace || !point_list) return GS_ERR_INVALID_ARGUMENT;
-  if (workspace_bytes < gs_bin_packed_workspace_bytes(num_rendered)) return GS_ERR_SCRATCH_TOO_SMALL;
   const size_t key_bytes = gs_align256((size_t)num_rendered * sizeof(uint64_t));
+  if (workspace_bytes < 2 * key_bytes + gs_align256(gs_sort_least_scratch_bytes(num_rendered)))
+    return GS_ERR_SCRATCH_TOO_SMALL;
   uint64_t* keys = reinterpret_cast<uint64_t*>(workspace);
   uint64_t* keys_alt = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(workspace) + key_bytes);
   void* scratch = reinterpret_cast<char*>(workspace) + 2 * key_bytes;

@@ -974,7 +974,6 @@ int bucket_layout(int32_t P, int32_t V, int64_t E, int32_t W, int32_t H, BucketL
   L.off_vals = take((size_t)P * 4);
   L.off_keys_alt = take((size_t)P * 4);
   L.off_vals_alt = take((size_t)P * 4);
-  L.off_sort = take(gs_sort_scratch_bytes(P));
   L.off_cw = take((size_t)V * 16);
   L.off_idx = take((size_t)V * 4);
   L.off_hist = take(nh * 4);
@@ -989,6 +988,8 @@ int bucket_layout(int32_t P, int32_t V, int64_t E, int32_t W, int32_t H, BucketL
   L.off_cinfo = take((size_t)L.nc2_max * 16);
   L.off_cnt2 = take((size_t)L.nc2_max * 64 * 4);
   L.off_tiles = take((size_t)L.num_tiles * 4);
+  // last, so that a workspace with less than the sort's fastest split needs serves too
+  L.off_sort = take(gs_sort_scratch_bytes(P));
   L.total = o;
   if (nh > 0x7fffffffULL) return GS_ERR_OVERFLOW;
   return GS_OK;
@@ -1033,7 +1034,7 @@ extern "C" int gs_bin_buckets(int32_t P, int32_t num_valid, int64_t num_entries,
   if ((reinterpret_cast<uintptr_t>(coverage) | reinterpret_cast<uintptr_t>(records) |
        reinterpret_cast<uintptr_t>(workspace)) & 15)
     return GS_ERR_MISALIGNED;
-  if (workspace_bytes < L.total) return GS_ERR_SCRATCH_TOO_SMALL;
+  if (workspace_bytes < L.off_sort + bucket_align(gs_sort_least_scratch_bytes(P))) return GS_ERR_SCRATCH_TOO_SMALL;
   if (depth_max < depth_min) return GS_ERR_INVALID_ARGUMENT;
   char* ws = static_cast<char*>(workspace);
   unsigned* keys = reinterpret_cast<unsigned*>(ws + L.off_keys);
@@ -1061,7 +1062,7 @@ extern "C" int gs_bin_buckets(int32_t P, int32_t num_valid, int64_t num_entries,
   hipLaunchKernelGGL(gs::bucket_depth_keys_kernel, dim3((P + 255) / 256), dim3(256), 0, s, P, cw, depths, depth_min,
                      keys, vals);
   int passes = 0;
-  st = gs_sort_pairs_u32_any(P, key_bits, keys, vals, keys_alt, vals_alt, ws + L.off_sort, L.off_cw - L.off_sort,
+  st = gs_sort_pairs_u32_any(P, key_bits, keys, vals, keys_alt, vals_alt, ws + L.off_sort, workspace_bytes - L.off_sort,
                              &passes, stream);
   if (st != GS_OK) return st;
   const int* order = passes % 2 ? vals_alt : vals;

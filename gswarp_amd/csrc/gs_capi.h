@@ -27,7 +27,9 @@ static inline int gs_bit_length(long long v) {
 // gs_sort_tile_segments whose workgroups take the tiles in the given order
 // (a permutation of the tiles, longest list first; null: tile order);
 // gs_sort_pairs_u32_any is gs_sort_pairs_u32 on the low key_bits bits in
-// however many passes are fastest, reported in *passes.
+// however many passes are fastest, reported in *passes;
+// gs_sort_least_scratch_bytes is the least scratch that the sorts of n keys
+// accept (gs_sort_scratch_bytes: what the fastest split needs).
 int gs_render_fwd_clear_ordered(int32_t image_width, int32_t image_height, int32_t num_points, int64_t num_rendered,
                                 const int32_t* ranges, const int32_t* point_list, const float* records,
                                 const float* background, int32_t compute_depth, float* out_color, float* out_depth,
@@ -38,3 +40,4 @@ int gs_sort_tile_segments_ordered(int64_t n, uint64_t* keys, uint64_t* keys_alt,
                                   int32_t* point_list, int32_t write_keys, const int32_t* order, void* stream);
 int gs_sort_pairs_u32_any(int64_t n, int32_t key_bits, uint32_t* keys, int32_t* values, uint32_t* keys_alt,
                           int32_t* values_alt, void* scratch, size_t scratch_bytes, int* passes, void* stream);
+size_t gs_sort_least_scratch_bytes(int64_t n);

@@ -352,7 +352,7 @@ static int sort_impl(int64_t n, int32_t lo_bit, int32_t key_bits, K* kin, K* kou
   if (passes_out) *passes_out = 0;
   if (n == 0 || key_bits == 0) return GS_OK;
   if (!kin || !kout || !scratch || (kValues && (!vin || !vout))) return GS_ERR_INVALID_ARGUMENT;
-  if (scratch_bytes < ((kDense.scratch_bytes(n) + 255) & ~(size_t)255)) return GS_ERR_SCRATCH_TOO_SMALL;
+  if (scratch_bytes < gs_sort_least_scratch_bytes(n)) return GS_ERR_SCRATCH_TOO_SMALL;
   const Plan plan = plan_for(n, key_bits, sizeof(K) + (kValues ? sizeof(int) : 0), scratch_bytes, kAnyDigits);
   unsigned* hist = reinterpret_cast<unsigned*>(scratch);
   unsigned* digit_totals = hist + ((size_t)plan.blocks(n) << plan.digit_bits);
@@ -384,6 +384,10 @@ static int sort_impl(int64_t n, int32_t lo_bit, int32_t key_bits, K* kin, K* kou
 extern "C" int gs_sort_num_passes(int32_t key_bits) { return gs_passes_for_bits(key_bits); }
 
 extern "C" size_t gs_sort_scratch_bytes(int64_t n) { return n <= 0 ? 0 : gs_sort::scratch_size(n); }
+
+size_t gs_sort_least_scratch_bytes(int64_t n) {
+  return n <= 0 ? 0 : (gs_sort::kDense.scratch_bytes(n) + 255) & ~(size_t)255;
+}
 
 int gs_sort_pairs_u32_any(int64_t n, int32_t key_bits, uint32_t* keys, int32_t* values, uint32_t* keys_alt,
                           int32_t* values_alt, void* scratch, size_t scratch_bytes, int* passes, void* stream) {

@@ -45,3 +45,24 @@ def test_lists_match_the_depth_tile_sort(count, width, height, device, monkeypat
     assert a.num_rendered == b.num_rendered >= count
     assert torch.equal(a.point_list, b.point_list)
     assert torch.equal(a.ranges, b.ranges)
+
+
+def test_workspace_of_the_least_size_serves(device, monkeypatch):
+    """The depth sort's fast split wants more scratch than 4096-key tiles; without it the lists are the same."""
+    from gswarp_amd import _lib
+
+    count = 20_000
+    scene = _pile(count, 130, 140, device)
+    monkeypatch.setattr(_pipeline, "DEPTH_TILE_MIN_PAIRS_PER_GAUSSIAN", 0)
+    monkeypatch.setattr(_pipeline, "BUCKET_SIZING", "always")
+    expected = gpu_forward(scene, options())["bins"].point_list
+    lib = _lib.load()
+    real = lib.gs_bin_buckets_workspace_bytes
+    least = ((count + 4095) // 4096 + 1) * 1024
+    short = int(lib.gs_sort_scratch_bytes(count)) - least
+    assert short > 0
+    monkeypatch.setattr(lib, "gs_bin_buckets_workspace_bytes", lambda *a: real(*a) - short)
+    assert torch.equal(gpu_forward(scene, options())["bins"].point_list, expected)
+    monkeypatch.setattr(lib, "gs_bin_buckets_workspace_bytes", lambda *a: real(*a) - short - 256)
+    with pytest.raises(RuntimeError):
+        gpu_forward(scene, options())
