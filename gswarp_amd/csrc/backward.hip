@@ -1545,11 +1545,11 @@ extern "C" size_t gs_render_bwd_workspace_bytes(int32_t image_width, int32_t ima
 }
 
 extern "C" int gs_render_bwd_ws(int32_t image_width, int32_t image_height, int32_t num_points,
-                             int64_t num_rendered, const int32_t* ranges,
-                             const int32_t* point_list, const float* records, const float* background,
-                             const float* out_alpha, const int32_t* n_contrib, const float* grad_color,
-                             const float* grad_depth, const float* grad_alpha, int32_t compute_depth,
-                             float* grad_gauss, const int32_t* tile_order, void* workspace,
+                                int64_t num_rendered, const int32_t* ranges,
+                                const int32_t* point_list, const float* records, const float* background,
+                                const float* out_alpha, const int32_t* n_contrib, const float* grad_color,
+                                const float* grad_depth, const float* grad_alpha, int32_t compute_depth,
+                                float* grad_gauss, const int32_t* tile_order, void* workspace,
                                 size_t workspace_bytes, void* stream) {
   if (image_width <= 0 || image_height <= 0 || (long long)image_width * image_height > 0x7fffffffLL)
     return GS_ERR_INVALID_ARGUMENT;

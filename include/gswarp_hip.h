@@ -295,7 +295,9 @@ int gs_duplicate_tiles(int32_t P, const int32_t* order, const int32_t* radii, co
  * gs_sort_pairs_u64 sorts (uint64 key, int32 value) pairs on the low
  * key_bits bits; gs_sort_keys_u64 sorts keys alone and gs_sort_pairs_u32
  * (uint32 key, int32 value) pairs, both on bits [lo_bit, lo_bit + key_bits)
- * (bits below lo_bit ride along).
+ * (bits below lo_bit ride along).  gs_sort_scratch_bytes(n) never falls as n
+ * grows; scratch of only one column of 256 counters per 4096 keys and one for
+ * the totals serves too, with a slower split of small sorts.
  * Replaces: binning_ops.py:337-343 and memory.py:586-600
  * (wp.utils.radix_sort_pairs on tile ids).
  */
