@@ -252,6 +252,14 @@ struct WalkSegment {
   float2* map_out = nullptr;     // kCompose: this segment's
 };
 
+// A segment's map of every pixel of the slice; the wave of every segment but
+// the front one stores it, whatever it walks.
+template <int kPix>
+__device__ __forceinline__ void store_maps(float2* map_out, const float (&a)[kPix], const float (&b)[kPix], int lane) {
+#pragma unroll
+  for (int k = 0; k < kPix; ++k) map_out[64 * k + lane] = make_float2(a[k], b[k]);
+}
+
 // One wave walks a slice of kPix blocks of 8x8 pixels, kCols blocks wide:
 // lane l owns pixel (l % 8, l / 8) of every block, block k lying at
 // ((k % kCols) 8, (k / kCols) 8) from the slice's origin.  Slice `sub` of a
@@ -381,7 +389,13 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
       }
     }
   }
-  if (max_lc <= lo) return;
+  if (max_lc <= lo) {
+    // Nothing to walk (slice_walk_kernel's length counts the pixels of T = 0
+    // too, which walk nothing here): the segment still has a map, the
+    // identity, which the segments in front of it read.
+    if constexpr (kSegment == SegmentMode::kCompose) store_maps<kPix>(seg.map_out, Ti, S, lane);
+    return;
+  }
   const int flush_comp = lane < kSlotFloats / 4 ? slot_component(lane >> 2) : -1;  // kCols == 2
   float* const col_raw = s_slot;  // kCols == 1
   const int raw_ofs = col_raw_offset(lane);
@@ -638,8 +652,7 @@ __device__ __forceinline__ void render_bwd_slice(const RenderBwdParams& p, int t
       walk(std::false_type{});
   }
   if constexpr (kSegment == SegmentMode::kCompose) {
-#pragma unroll
-    for (int k = 0; k < kPix; ++k) seg.map_out[64 * k + lane] = make_float2(Ti[k], S[k]);
+    store_maps<kPix>(seg.map_out, Ti, S, lane);
     return;
   }
   if (kCols > 1 && slot_gid >= 0) flush_slot(s_slot, slot_gid, lane, flush_comp, p.grad_gauss);

@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from gswarp_amd import _lib, configs
+from helpers import gpu_forward, options
 from test_gpu_parity import _check_backward
 
 
@@ -37,6 +38,48 @@ def _pile(count: int, side: int, sigma_px: float, device) -> dict:
 def test_quadrant_segments_match_oracle(count, device):
     assert _lib.load().gs_render_bwd_workspace_bytes(16, 16, count, count) > 0
     _check_backward(_pile(count, 16, 1.5, device))
+
+
+def _walks(scene, limit: int, opaque_limit: int, device):
+    """(segmented, whole) render gradients, (N, 10), of a scene whose blocks of 8 x 8 pixels are given walks
+    of at most `limit` entries, but for one pixel each of at most `opaque_limit` whose alpha is 1.  The
+    segmented walk's workspace is filled with NaN."""
+    out = gpu_forward(scene, options())
+    pre, bins, res = out["pre"], out["bins"], out["res"]
+    H, W, N, R = scene["height"], scene["width"], scene["means3D"].shape[0], bins.num_rendered
+    n_contrib = res.n_contrib.view(H, W).clamp(max=limit)
+    alpha = res.alpha.clone()
+    at = (slice(3, None, 8), slice(5, None, 8))
+    n_contrib[at] = res.n_contrib.view(H, W)[at].clamp(max=opaque_limit)
+    alpha[0][at] = 1.0
+    g = torch.Generator().manual_seed(9)
+    grads = [torch.randn(c, H, W, generator=g).to(device) for c in (3, 1, 1)]
+    lib = _lib.load()
+    size = lib.gs_render_bwd_workspace_bytes(W, H, N, R)
+    assert size > 0
+    sums = []
+    for ws in (torch.full((size // 4,), float("nan"), device=device), None):
+        acc = torch.zeros((N, 10), device=device)
+        lib.call("gs_render_bwd_ws", W, H, N, R, bins.ranges.data_ptr(), bins.point_list.data_ptr(),
+                 pre.records.data_ptr(), scene["bg"].data_ptr(), alpha.data_ptr(), n_contrib.data_ptr(),
+                 *(t.data_ptr() for t in grads), 1, acc.data_ptr(), None, _lib.ptr(ws), size if ws is not None else 0,
+                 torch.cuda.current_stream(device).cuda_stream)
+        sums.append(acc)
+    torch.cuda.synchronize()
+    return sums
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,side,sigma,pixels", [(400, 16, 6.0, "quadrants"), (400, 67, 40.0, "halves")])
+@pytest.mark.parametrize("limit", [0, 1, 90, 128, 129, 300])
+def test_opaque_pixel_with_the_longest_walk(count, side, sigma, pixels, limit, device):
+    """A pixel of alpha 1 blends nothing: where it alone has entries in the last segments, those segments
+    pass the other pixels' state on unchanged."""
+    segmented, whole = _walks(_pile(count, side, sigma, device), limit, 1 << 30, device)
+    # a pixel's state is a product and a sum over at most 300 entries, each rounded to 2^-24 of it, and a
+    # Gaussian's sum has at most a few hundred terms of either sign
+    tol = 1e-4 * whole.abs().amax(dim=0, keepdim=True) + 1e-12
+    assert bool(((segmented - whole).abs() <= tol).all())
 
 
 @pytest.mark.gpu
