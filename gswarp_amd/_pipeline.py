@@ -921,9 +921,10 @@ def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, gra
         if bins.num_rendered != 0:
             ws_bytes = int(lib.gs_render_bwd_workspace_bytes(W, H, P, bins.num_rendered))
             ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=device) if ws_bytes > 0 else None
+            background = inputs.background.to(device)  # held: a copy on the device is freed with its last reference
             with _stage("render_bwd"):
                 lib.call("gs_render_bwd_ws", W, H, P, bins.num_rendered, bins.address("ranges"),
-                         bins.address("point_list"), records_at, _address(inputs.background.to(device), copies),
+                         bins.address("point_list"), records_at, _address(background, copies),
                          _address(alpha, copies), n_contrib_at, _address_or_none(grad_color, copies),
                          _address_or_none(grad_depth, copies), _address_or_none(grad_alpha, copies),
                          int(bool(options.compute_depth)), grad_gauss_at, bins.address("tile_order"), _lib.ptr(ws),
