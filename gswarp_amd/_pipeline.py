@@ -899,6 +899,9 @@ def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, gra
         return (torch.zeros((0, 3), dtype=torch.float32, device=device), grad_colors,
                 torch.empty_like(inputs.opacities), torch.zeros_like(means), grad_cov3d,
                 torch.empty_like(inputs.sh), torch.zeros_like(inputs.scales), torch.zeros_like(inputs.rotations))
+    has_sh = inputs.sh.numel() != 0
+    if has_sh and inputs.sh.numel() % (NUM_CHANNELS * P):
+        raise RuntimeError(f"sh of {inputs.sh.numel()} values does not hold whole RGB coefficients of {P} Gaussians")
     with _device_guard(device), _workspace.device_lock(device):
         if forward_state is None:
             # Second backward of a retained graph: rebuild the forward state.
@@ -929,8 +932,7 @@ def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, gra
                          _address_or_none(grad_depth, copies), _address_or_none(grad_alpha, copies),
                          int(bool(options.compute_depth)), grad_gauss_at, bins.address("tile_order"), _lib.ptr(ws),
                          ws_bytes, stream)
-        has_sh = inputs.sh.numel() != 0
-        K = inputs.sh.numel() // (3 * P) if has_sh else 0
+        K = inputs.sh.numel() // (NUM_CHANNELS * P) if has_sh else 0
         grad_sh = torch.empty((P, K, NUM_CHANNELS), **f) if has_sh else torch.empty_like(inputs.sh)
         grad_means3d = torch.empty((P, 3), **f)
         grad_means2d = torch.empty((P, 3), **f)
