@@ -803,7 +803,7 @@ def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torc
     proj_2d = torch.empty((P, 2), dtype=f32, device=device)
     conic_2d = torch.empty((P, 3), dtype=f32, device=device)
     conic_2d_inv = torch.empty((P, 3), dtype=f32, device=device)
-    pre = ArenaPreprocessOutputs(radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode, arena)
+    pre = ArenaPreprocessOutputs.within(arena, radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode)
     copies = []
     tanfovx, tanfovy = float(inputs.tan_fovx), float(inputs.tan_fovy)
     radii_at, records_at, tiles_at = radii.data_ptr(), arena.address("records"), arena.address("tiles_touched")
@@ -848,7 +848,7 @@ def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torc
         _workspace.note_pairs(device, R)
         if result[4]:
             layout = KeyLayout(result[1], result[2], result[3])
-            bins = ArenaBinningState(grid_x, grid_y, point_list[:R], R, layout, arena, bool(result[5]))
+            bins = ArenaBinningState.within(arena, grid_x, grid_y, point_list[:R], R, layout, bool(result[5]))
         else:
             depth_range = slot[1] & 0xFFFFFFFFFFFFFFFF
             # declined: release the provisioned buffers before the exact-size binning allocates its own
@@ -868,7 +868,7 @@ def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torc
         images = RenderImages(_f32c(inputs.background), color, depth, alpha, arena.view("n_contrib"), compute_depth)
         aux = render(pre, bins, inputs.background, H, W, options, flow=flow, images=images, grad_clear=grad_gauss).aux
     return ForwardResult(R, color, depth, alpha, radii, proj_2d, conic_2d, conic_2d_inv,
-                         ArenaForwardState(pre, bins, arena, grad_gauss), aux)
+                         ArenaForwardState.within(arena, pre, bins, grad_gauss), aux)
 
 
 def _depths_or_none(pre: PreprocessOutputs) -> int | None:

@@ -7,7 +7,7 @@ separate points_xy / conic_opacity / features / depths arrays.
 
 from __future__ import annotations
 
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, fields
 
 import torch
 
@@ -117,11 +117,12 @@ class ForwardState:
 
 class StateArena:
     """One device allocation for the arrays that a typed forward keeps for its
-    backward and shows to nobody else.  The stages and the backward need
-    their addresses only; a tensor view is made when one is asked for, which
-    spares an allocation or a view of each on every call."""
+    backward.  The stages and the backward need their addresses only; a
+    tensor view is made when one is asked for, which spares an allocation or a
+    view of each on every call.  A view that is kept keeps the whole
+    allocation (a clone does not)."""
 
-    __slots__ = ("buffer", "base", "spans")
+    __slots__ = ("buffer", "spans")
 
     def __init__(self, spans, device: torch.device):
         """spans: (name, dtype, shape, bytes) of each array; every array starts on a 256-byte boundary."""
@@ -131,26 +132,66 @@ class StateArena:
             self.spans[name] = (at, dtype, shape, nbytes)
             at += (nbytes + 255) & ~255
         self.buffer = torch.empty((at,), dtype=torch.uint8, device=device)
-        self.base = self.buffer.data_ptr()
 
     def address(self, name: str) -> int:
-        return self.base + self.spans[name][0]
+        return self.buffer.data_ptr() + self.spans[name][0]
 
     def view(self, name: str) -> torch.Tensor:
         at, dtype, shape, nbytes = self.spans[name]
         return self.buffer[at:at + nbytes].view(dtype).view(shape)
 
 
-def _arena_field(name: str):
-    return property(lambda self: self.arena.view(name) if name in self.arena.spans else None)
+def _arena_field(name: str) -> property:
+    """A dataclass field whose array lies in the arena until another is set."""
+
+    def get(self):
+        if name not in self.own:
+            self.own[name] = self.arena.view(name) if name in self.arena.spans else None
+        return self.own[name]
+
+    def put(self, value):
+        self.own[name] = value
+
+    return property(get, put)
 
 
-class ArenaPreprocessOutputs:
+class _InArena:
+    """What makes a state dataclass one whose _arena_field arrays lie in
+    ``arena``; ``own`` holds the views made of them and what was set in their
+    place.  To its holder it is the dataclass ``plain``: it is made by
+    ``within``, or by the dataclass's own constructor (dataclasses.replace)
+    with every array given; copies and pickles are plain ones."""
+
+    __slots__ = ()
+    plain: type
+
+    def __new__(cls, *args, **kwargs):
+        self = super().__new__(cls)
+        self.arena, self.own = None, {}
+        return self
+
+    def address(self, name: str) -> int | None:
+        if self.arena is None or name in self.own or name not in self.arena.spans:
+            return super().address(name)
+        return self.arena.address(name)
+
+    def _values(self) -> dict:
+        return {f.name: getattr(self, f.name) for f in fields(self)}
+
+    def __copy__(self):
+        return self.plain(**self._values())
+
+    def __reduce__(self):
+        # arrays of different types in one storage cannot be saved together
+        values = [v.clone() if k in self.own and v is not None else v for k, v in self._values().items()]
+        return self.plain, tuple(values)
+
+
+class ArenaPreprocessOutputs(_InArena, PreprocessOutputs):
     """PreprocessOutputs whose arrays, but for the four that the forward returns, lie in an arena."""
 
-    __slots__ = ("radii", "proj_2d", "conic_2d", "conic_2d_inv", "coverage_mode", "arena")
-    geom = None
-    scan_state = None  # the arena's state has served its scan
+    __slots__ = ("arena", "own")
+    plain = PreprocessOutputs
     depths = _arena_field("depths")
     tiles_touched = _arena_field("tiles_touched")
     records = _arena_field("records")
@@ -158,50 +199,58 @@ class ArenaPreprocessOutputs:
     coverage = _arena_field("coverage")
     band_store = _arena_field("band_store")
 
-    def __init__(self, radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode: int, arena: StateArena):
+    @classmethod
+    def within(cls, arena: StateArena, radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode: int):
+        self = cls.__new__(cls)
+        self.arena = arena
         self.radii, self.proj_2d, self.conic_2d, self.conic_2d_inv = radii, proj_2d, conic_2d, conic_2d_inv
         self.coverage_mode = coverage_mode
-        self.arena = arena
+        self.geom = None
+        self.scan_state = None  # the arena's has served its scan
+        return self
 
-    def address(self, name: str) -> int | None:
-        return self.arena.address(name) if name in self.arena.spans else None
 
-
-class ArenaBinningState(BinningState):
+class ArenaBinningState(_InArena, BinningState):
     """BinningState of the packed binning launched with the read-back, its ranges and tile order in an arena."""
 
-    __slots__ = ("arena", "has_order")
+    __slots__ = ("arena", "own")
+    plain = BinningState
     ranges = _arena_field("ranges")
-    tile_order = property(lambda self: self.arena.view("tile_order") if self.has_order else None)
+    tile_order = _arena_field("tile_order")
 
-    def __init__(self, grid_x, grid_y, point_list, num_rendered, key_layout, arena: StateArena, rendered: bool):
+    @classmethod
+    def within(cls, arena: StateArena, grid_x: int, grid_y: int, point_list, num_rendered: int, key_layout: KeyLayout,
+               rendered: bool):
+        self = cls.__new__(cls)
+        self.arena = arena
         self.grid_x, self.grid_y = grid_x, grid_y
         self.point_list, self.num_rendered, self.key_layout = point_list, num_rendered, key_layout
         self.sorted_keys = self.buffer = None
-        self.arena, self.rendered, self.has_order = arena, rendered, rendered
+        self.rendered = rendered
+        if not rendered:
+            self.tile_order = None  # until a render writes it
+        return self
 
     def ensure_tile_order(self, num_tiles: int) -> None:
-        self.has_order = True
-
-    def address(self, name: str) -> int | None:
-        if name == "point_list":
-            return self.point_list.data_ptr()
-        if name == "tile_order" and not self.has_order:
-            return None
-        return self.arena.address(name)
+        if self.arena is None:
+            super().ensure_tile_order(num_tiles)
+        elif self.own.get("tile_order", self) is None:
+            del self.own["tile_order"]  # the arena's
 
 
-class ArenaForwardState:
+class ArenaForwardState(_InArena, ForwardState):
     """ForwardState with n_contrib in an arena."""
 
-    __slots__ = ("preprocess", "binning", "arena", "grad_gauss")
+    __slots__ = ("arena", "own")
+    plain = ForwardState
     n_contrib = _arena_field("n_contrib")
 
-    def __init__(self, preprocess, binning, arena: StateArena, grad_gauss):
-        self.preprocess, self.binning, self.arena, self.grad_gauss = preprocess, binning, arena, grad_gauss
-
-    def address(self, name: str) -> int:
-        return self.arena.address(name)
+    @classmethod
+    def within(cls, arena: StateArena, preprocess: PreprocessOutputs, binning: BinningState, grad_gauss):
+        self = cls.__new__(cls)
+        self.arena = arena
+        self.preprocess, self.binning, self.grad_gauss = preprocess, binning, grad_gauss
+        return self
 
 
 @dataclass(slots=True)

@@ -4,9 +4,12 @@ and the same gradients up to the order of the float atomics."""
 
 from __future__ import annotations
 
+import copy
+
 import pytest
 import torch
 
+from helpers import options, raster_inputs
 from gswarp_amd import _pipeline, _validation, _workspace, configs, rasterizer, rasterizer_flow
 from gswarp_amd.methods import mip_3dgs
 
@@ -98,6 +101,28 @@ def test_arena_forward_equals_general(form, config, hint, device, monkeypatch):
         assert a.shape == b.shape
         # the atomics' order: a few hundred float32 additions per element
         assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max()) + 1e-12
+
+
+def test_backward_from_a_copied_state(device):
+    """The copy is on its own: the state it was made from is gone, and its memory overwritten, by the backward."""
+    scene = configs.make_scene(2, seed=3, count=5_000, width=120, height=90, device=device)
+    inputs, opts = raster_inputs(scene), options()
+    _workspace.note_pairs(device, 5_000)
+    upstream = torch.randn(3, 90, 120, generator=torch.Generator().manual_seed(1)).to(device)
+
+    def grads(copied: bool):
+        result = _pipeline.forward(inputs, opts)
+        state = result.state
+        if copied:
+            state = copy.deepcopy(state)
+            result.state.binning.arena.buffer.fill_(255)
+        return _pipeline.backward(inputs, result.radii, result.alpha, upstream, None, None, None, None, None, opts,
+                                  state)
+
+    for a, b in zip(grads(True), grads(False)):
+        assert a.shape == b.shape
+        if b.numel():  # the atomics' order
+            assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max()) + 1e-12
 
 
 def test_first_forward_takes_the_general_course(device):
