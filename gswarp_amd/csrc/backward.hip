@@ -735,11 +735,31 @@ __global__ __launch_bounds__(64) void render_bwd_whole_kernel(RenderBwdParams p)
 // which saves their maps, measured the same.
 constexpr int kSegmentEntries = 128;
 
-// Most segments of a walk: more where there are fewer tiles, since each
-// costs a wave per slice that returns at once when its walk is shorter (about
-// 1.5 us per 10,000).  640x640: 16 segments 182 us, 8 207 us; 800x800, 300k
-// Gaussians: 8 segments 156 us, 16 176 us.
-static int max_segments(int64_t num_tiles) { return num_tiles <= 1024 ? 32 : num_tiles <= 2048 ? 16 : 8; }
+// Most segments of a walk, 1 for none.  Each costs a wave per slice in both
+// launches that returns at once when its walk is shorter (2.1 us per 10,000), so
+// - more where there are fewer tiles.  640x640: 16 segments 182 us, 8 207 us;
+//   800x800, 300k Gaussians: 8 segments 156 us, 16 176 us;
+// - no more than a list of kSegmentListsPerMean times the mean length fills,
+//   but where there are too few tiles for empty waves to matter.  How uneven the
+//   lists are is not known here: a small object's are 10 to 18 times the mean
+//   where they are longest, those of a scene that fills its image twice.  The
+//   kernels in us, whole / cut for 16 / for 32 / for 64 times the mean / without
+//   this limit:
+//     512x512, splats of two tiles all over it: 1000 6 / 6 / 6 / 10 / 60,
+//       10,000 15 / 17 / 19 / 24 / 60, 30,000 30 / 34 / 40 / 60 / 60
+//     on a sixteenth of it: 1000 10 / 10 / 10 / 15 / 59,
+//       10,000 58 / 50 / 46 / 46 / 60, 30,000 157 / 76 / 76 / 81 / 81
+//     on a hundredth: 10,000 254 / 160 / 111 / 87 / 84.
+constexpr int64_t kSegmentListsPerMean = 32;
+
+static int max_segments(int64_t num_tiles, int64_t num_rendered) {
+  const int64_t most = num_tiles <= 1024 ? 32 : num_tiles <= 2048 ? 16 : 8;
+  const int64_t unit = num_tiles * kSegmentEntries;
+  const int64_t needed = (kSegmentListsPerMean * num_rendered + unit - 1) / unit;
+  const int64_t few = 128 / num_tiles;
+  const int64_t n = needed > few ? needed : few;
+  return (int)(n > most ? most : n > 1 ? n : 1);
+}
 
 // Entries per segment (a multiple of 64, whole batches) of a walk.
 __device__ __forceinline__ int segment_length(int walk, int max_segments) {
@@ -831,7 +851,7 @@ __global__ __launch_bounds__(64, 6) void render_bwd_segments_kernel(RenderBwdPar
 constexpr int64_t kSegmentContendedPairsPerPoint = 12;
 
 static int segment_pixels(int64_t num_tiles, int64_t num_rendered, int64_t num_points) {
-  if (num_tiles > 2600) return 0;
+  if (num_tiles > 2600 || max_segments(num_tiles, num_rendered) == 1) return 0;
   if (num_rendered > kSegmentContendedPairsPerPoint * num_points) return num_tiles <= 1600 ? 2 : 0;
   if (num_tiles <= 1600 || num_rendered > kWholeTilePairsPerPoint * num_points) return 1;
   return num_rendered <= 500000 ? 1 : num_rendered <= 1250000 ? 2 : 0;
@@ -839,21 +859,21 @@ static int segment_pixels(int64_t num_tiles, int64_t num_rendered, int64_t num_p
 
 // The workspace of the segmented walk: the maps of every quadrant (or, at
 // two pixels per lane, half), then the walk lengths.
-static size_t segment_maps_bytes(int64_t num_tiles) {
-  return (size_t)num_tiles * (max_segments(num_tiles) - 1) * kTilePixels * sizeof(float2);
+static size_t segment_maps_bytes(int64_t num_tiles, int64_t num_rendered) {
+  return (size_t)num_tiles * (max_segments(num_tiles, num_rendered) - 1) * kTilePixels * sizeof(float2);
 }
 
-static size_t segment_workspace_bytes(int64_t num_tiles) {
-  return segment_maps_bytes(num_tiles) + (size_t)num_tiles * 4 * sizeof(int);
+static size_t segment_workspace_bytes(int64_t num_tiles, int64_t num_rendered) {
+  return segment_maps_bytes(num_tiles, num_rendered) + (size_t)num_tiles * 4 * sizeof(int);
 }
 
 template <bool kDepth, int kPix>
 static void launch_render_bwd_segments(const RenderBwdParams& p, char* workspace, hipStream_t s) {
   constexpr int kSubs = 4 / kPix;
   float2* const maps = reinterpret_cast<float2*>(workspace);
-  int* const walk = reinterpret_cast<int*>(workspace + segment_maps_bytes(p.num_tiles));
+  int* const walk = reinterpret_cast<int*>(workspace + segment_maps_bytes(p.num_tiles, p.num_rendered));
   const int units = xcd_grid(kSubs * p.num_tiles);
-  const int segments = max_segments(p.num_tiles);
+  const int segments = max_segments(p.num_tiles, p.num_rendered);
   hipLaunchKernelGGL((slice_walk_kernel<kPix>), dim3((kSubs * p.num_tiles + 3) / 4), dim3(256), 0, s, p, walk);
   hipLaunchKernelGGL((render_bwd_compose_kernel<kDepth, kPix>), dim3(units * (segments - 1)), dim3(64), 0, s, p, walk,
                      maps, segments);
@@ -1554,7 +1574,7 @@ extern "C" size_t gs_render_bwd_workspace_bytes(int32_t image_width, int32_t ima
   if (image_width <= 0 || image_height <= 0 || num_points <= 0 || num_rendered <= 0) return 0;
   const int64_t tiles = ((int64_t)(image_width + gs::kBlockX - 1) / gs::kBlockX) *
                         ((image_height + gs::kBlockY - 1) / gs::kBlockY);
-  return gs::segment_pixels(tiles, num_rendered, num_points) ? gs::segment_workspace_bytes(tiles) : 0;
+  return gs::segment_pixels(tiles, num_rendered, num_points) ? gs::segment_workspace_bytes(tiles, num_rendered) : 0;
 }
 
 extern "C" int gs_render_bwd_ws(int32_t image_width, int32_t image_height, int32_t num_points,

@@ -99,3 +99,30 @@ def test_workspace_only_where_the_walk_is_cut():
     assert not needs(640, 640, 1000, 0) and not needs(0, 640, 1000, 1000)
     # 64 (a, b) pairs for each of a quadrant's segments but the first, and its length
     assert lib.gs_render_bwd_workspace_bytes(16, 16, 10, 10) == 4 * (31 * 64 * 8 + 4)
+
+
+def test_no_more_segments_than_the_lists_fill():
+    """Segments of 128 entries for lists of 32 times the mean length, but where there are fewer than 128 tiles."""
+    lib = _lib.load()
+    size = lib.gs_render_bwd_workspace_bytes
+    cut = lambda tiles, segments: tiles * ((segments - 1) * 256 * 8 + 4 * 4)
+    assert size(512, 512, 3000, 4096) == 0  # 1024 tiles, mean 4
+    assert size(512, 512, 3000, 4097) == cut(1024, 2)
+    assert size(512, 512, 30_000, 4096 * 31) == cut(1024, 31)
+    assert size(512, 512, 1_000_000, 4096 * 100) == cut(1024, 32)
+    assert size(800, 800, 100, 200) == 0 and size(800, 800, 100_000, 10_001) == cut(2500, 2)
+    assert size(176, 176, 100, 200) == 0  # 121 tiles
+    assert size(128, 128, 100, 200) == cut(64, 2) and size(32, 32, 100, 200) == cut(4, 32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [500, 1500])
+def test_segments_longer_than_128_entries_match_oracle(count, device):
+    """A small object: its lists are longer than the cut is made for."""
+    scene = _pile(count, 256, 3.0, device)
+    scene["means3D"][:, :2] *= 0.05
+    out = gpu_forward(scene, options())["bins"]
+    longest = int((out.ranges[:, 1] - out.ranges[:, 0]).max())
+    segments = _lib.load().gs_render_bwd_workspace_bytes(256, 256, count, out.num_rendered) // (256 * 2048) + 1
+    assert 1 < segments and longest > 128 * segments
+    _check_backward(scene)
