@@ -562,9 +562,15 @@ __global__ __launch_bounds__(64) void render_fwd_block_kernel(RenderFwdParams p)
 // pairs, 131 and 165) or with 4 to 12 pairs per Gaussian (500k mid-sized splats on
 // 700x700 198 and 117).  Above 12 pairs per Gaussian opaque pixels end the
 // walks early and the records' loads weigh more (640x480 37 and 47); above
-// 2600 tiles the quadrants fill the chip (300k on 1280x720 79 and 95).
+// 2600 tiles the quadrants fill the chip (300k on 1280x720 79 and 95).  With
+// less than 4 pairs a tile there is little to walk, and above 512 tiles the
+// sixteen waves of each cost more than they save: 100 and 1000 splats of two
+// tiles on 512x512 5 and 7, 5 and 8, on 640x640 6 and 9, 6 and 10, on 800x800 7
+// and 12, 7 and 13 (but 5.6 and 4.7 on 256x256).  Above, lists of even length are
+// up to 8 us slower in blocks and those of small objects up to 50 faster.
 static bool blocks_pay(int64_t num_tiles, int64_t num_rendered, int64_t num_points) {
   if (num_tiles > 2600 || num_rendered > 12 * num_points) return false;
+  if (num_tiles > 512 && num_rendered < 4 * num_tiles) return false;
   return num_tiles <= 1600 || num_rendered <= 1250000 || num_rendered > 4 * num_points;
 }
 

@@ -45,6 +45,15 @@ def test_block_edges_match_oracle(width, height, device):
     _check_forward(scene, options(compute_depth=False))
 
 
+@pytest.mark.parametrize("count", [150, 700])
+def test_light_images_match_oracle(count, device):
+    """Both sides of the least number of pairs that blocks take on more than 512 tiles."""
+    scene = _pile(count, 400, 336, (0.05, 0.9), device)
+    _check_forward(scene, options())
+    pairs = gpu_forward(scene, options())["bins"].num_rendered
+    assert (pairs < 4 * 25 * 21) == (count == 150)
+
+
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_non_finite_colour_stays_with_its_pixels(value, device):
     """A step evaluates four records at a pixel; one that the pixel does not blend adds nothing, whatever its colour."""
