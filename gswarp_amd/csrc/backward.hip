@@ -1593,7 +1593,7 @@ extern "C" int gs_render_bwd_ws(int32_t image_width, int32_t image_height, int32
   if (reinterpret_cast<uintptr_t>(records) & 15) return GS_ERR_MISALIGNED;
   if (reinterpret_cast<uintptr_t>(workspace) & 7) return GS_ERR_MISALIGNED;
   const size_t needed = gs_render_bwd_workspace_bytes(image_width, image_height, num_points, num_rendered);
-  if (workspace && workspace_bytes < needed) return GS_ERR_INVALID_ARGUMENT;
+  if (workspace && workspace_bytes < needed) return GS_ERR_SCRATCH_TOO_SMALL;
   gs::RenderBwdParams p;
   p.W = image_width;
   p.H = image_height;

@@ -115,6 +115,18 @@ def test_no_more_segments_than_the_lists_fill():
     assert size(128, 128, 100, 200) == cut(64, 2) and size(32, 32, 100, 200) == cut(4, 32)
 
 
+def test_short_workspace_is_refused():
+    """As short scratch is by the sorts and the binning, before anything is launched."""
+    lib = _lib.load()
+    size = lib.gs_render_bwd_workspace_bytes(64, 64, 1000, 5000)
+    at = 4096  # never read: the call returns before its launches
+    call = lambda ws, nbytes: lib.gs_render_bwd_ws(64, 64, 1000, 5000, at, at, at, at, at, at, at, at, at, 1, at, None,
+                                                   ws, nbytes, None)
+    assert size > 0 and call(at, size - 1) == -3 and call(at, 0) == -3
+    assert "scratch" in lib.status_string(-3)
+    assert call(at + 4, size) not in (0, -3)  # misaligned
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("count", [500, 1500])
 def test_segments_longer_than_128_entries_match_oracle(count, device):
