@@ -877,12 +877,6 @@ def _depths_or_none(pre: PreprocessOutputs) -> int | None:
     return pre.depths.data_ptr() if pre.depths.numel() == pre.radii.numel() and pre.radii.numel() > 0 else None
 
 
-def _f32c_or_none(t: torch.Tensor | None) -> torch.Tensor | None:
-    """Contiguous fp32 upstream gradient, or None (the kernels read an absent
-    gradient as zero)."""
-    return None if t is None else _f32c(t)
-
-
 def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, grad_color, grad_depth, grad_alpha,
              grad_proj_2d, grad_conic_2d, grad_conic_2d_inv, options: ExecutionOptions,
              forward_state: ForwardState | None, *, flow_double: bool = False):
