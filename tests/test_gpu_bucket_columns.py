@@ -6,7 +6,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gswarp_amd import _pipeline, configs
+from gswarp_amd import _lib, _pipeline, configs
 from helpers import gpu_forward, options
 
 pytestmark = pytest.mark.gpu
@@ -45,6 +45,42 @@ def test_lists_match_the_depth_tile_sort(count, width, height, device, monkeypat
     assert a.num_rendered == b.num_rendered >= count
     assert torch.equal(a.point_list, b.point_list)
     assert torch.equal(a.ranges, b.ranges)
+
+
+@pytest.mark.parametrize("count", [5000, 1_572_864, 1_572_865])
+def test_depth_order_in_wide_digits(count, device, monkeypatch):
+    """Depths of 25 to 27 bits take a digit pass less in 9-bit digits, up to 1.5M Gaussians; equal depths keep
+    their order."""
+    width, height = 300, 260
+    scene = _pile(count, width, height, device)
+    g = torch.Generator().manual_seed(count + 1)
+    depth = 2.0 + 7.0 * torch.rand(count, generator=g)
+    depth[::7] = depth[0]
+    depth = depth.to(device)
+    scene["means3D"] *= (depth / 4.0)[:, None]  # the same place in the image
+    scene["means3D"][:, 2] = depth - 4.0
+    scene["scales"] *= (depth / 4.0)[:, None]
+    monkeypatch.setattr(_pipeline, "DEPTH_TILE_MIN_PAIRS_PER_GAUSSIAN", 0)
+    monkeypatch.setattr(_pipeline, "BUCKET_SIZING", "always")
+    outs = {}
+    for flow in ("buckets", "depth_tile"):
+        monkeypatch.setattr(_pipeline, "HEAVY_DATAFLOW", flow)
+        print(f"[wide digits] N={count} {flow}", flush=True)
+        outs[flow] = gpu_forward(scene, options())
+    pre = outs["buckets"]["pre"]
+    bits = pre.depths[pre.radii > 0].view(torch.int32)
+    assert (int(bits.max()) - int(bits.min()) + 1).bit_length() in (25, 26, 27)
+    a, b = outs["buckets"]["bins"], outs["depth_tile"]["bins"]
+    assert a.num_rendered == b.num_rendered >= count
+    assert torch.equal(a.point_list, b.point_list) and torch.equal(a.ranges, b.ranges)
+    # scratch for 8-bit digits of 4096-key tiles only: the narrow digits, a pass more
+    lib = _lib.load()
+    real = lib.gs_bin_buckets_workspace_bytes
+    short = int(lib.gs_sort_scratch_bytes(count)) - ((count + 4095) // 4096 + 1) * 1024
+    assert short > 0
+    monkeypatch.setattr(_pipeline, "HEAVY_DATAFLOW", "buckets")
+    monkeypatch.setattr(lib, "gs_bin_buckets_workspace_bytes", lambda *args: real(*args) - short)
+    assert torch.equal(gpu_forward(scene, options())["bins"].point_list, b.point_list)
 
 
 def test_workspace_of_the_least_size_serves(device, monkeypatch):

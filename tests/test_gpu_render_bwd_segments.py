@@ -40,18 +40,11 @@ def test_quadrant_segments_match_oracle(count, device):
     _check_backward(_pile(count, 16, 1.5, device))
 
 
-def _walks(scene, limit: int, opaque_limit: int, device):
-    """(segmented, whole) render gradients, (N, 10), of a scene whose blocks of 8 x 8 pixels are given walks
-    of at most `limit` entries, but for one pixel each of at most `opaque_limit` whose alpha is 1.  The
-    segmented walk's workspace is filled with NaN."""
-    out = gpu_forward(scene, options())
-    pre, bins, res = out["pre"], out["bins"], out["res"]
+def _sums(scene, out, alpha, n_contrib):
+    """(segmented, whole) render gradients, (N, 10), of a forward; the segmented walk's workspace is filled
+    with NaN."""
+    pre, bins, device = out["pre"], out["bins"], alpha.device
     H, W, N, R = scene["height"], scene["width"], scene["means3D"].shape[0], bins.num_rendered
-    n_contrib = res.n_contrib.view(H, W).clamp(max=limit)
-    alpha = res.alpha.clone()
-    at = (slice(3, None, 8), slice(5, None, 8))
-    n_contrib[at] = res.n_contrib.view(H, W)[at].clamp(max=opaque_limit)
-    alpha[0][at] = 1.0
     g = torch.Generator().manual_seed(9)
     grads = [torch.randn(c, H, W, generator=g).to(device) for c in (3, 1, 1)]
     lib = _lib.load()
@@ -69,17 +62,57 @@ def _walks(scene, limit: int, opaque_limit: int, device):
     return sums
 
 
+def _walks(scene, limit: int, device):
+    """_sums of a scene whose blocks of 8 x 8 pixels are given walks of at most `limit` entries, but for one
+    pixel each whose alpha is 1."""
+    out = gpu_forward(scene, options())
+    n_contrib = out["res"].n_contrib.view(scene["height"], scene["width"]).clamp(max=limit)
+    alpha = out["res"].alpha.clone()
+    at = (slice(3, None, 8), slice(5, None, 8))
+    n_contrib[at] = out["res"].n_contrib.view_as(n_contrib)[at]
+    alpha[0][at] = 1.0
+    return _sums(scene, out, alpha, n_contrib)
+
+
+def _assert_close(segmented, whole):
+    # a pixel's state is a product and a sum over a few hundred entries, each rounded to 2^-24 of it, and a
+    # Gaussian's sum has at most a few hundred terms of either sign
+    tol = 1e-4 * whole.abs().amax(dim=0, keepdim=True) + 1e-12
+    assert bool(((segmented - whole).abs() <= tol).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("count,side,sigma,pixels", [(400, 16, 6.0, "quadrants"), (400, 67, 40.0, "halves")])
 @pytest.mark.parametrize("limit", [0, 1, 90, 128, 129, 300])
 def test_opaque_pixel_with_the_longest_walk(count, side, sigma, pixels, limit, device):
     """A pixel of alpha 1 blends nothing: where it alone has entries in the last segments, those segments
     pass the other pixels' state on unchanged."""
-    segmented, whole = _walks(_pile(count, side, sigma, device), limit, 1 << 30, device)
-    # a pixel's state is a product and a sum over at most 300 entries, each rounded to 2^-24 of it, and a
-    # Gaussian's sum has at most a few hundred terms of either sign
-    tol = 1e-4 * whole.abs().amax(dim=0, keepdim=True) + 1e-12
-    assert bool(((segmented - whole).abs() <= tol).all())
+    _assert_close(*_walks(_pile(count, side, sigma, device), limit, device))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,side,sigma,pixels", [(700, 16, 2.0, "quadrants"), (1200, 67, 25.0, "halves")])
+def test_pixels_of_a_block_end_in_different_segments(count, side, sigma, pixels, device):
+    """Opaque splats in front cover a column of each of the first tile's blocks: their pixels end after some tens of
+    entries, beside pixels whose walks reach the list's end."""
+    scene = _pile(count, side, sigma, device)
+    g = torch.Generator().manual_seed(count)
+    pixel = 8.0 * scene["tanfovx"] / side
+    front = torch.rand(120, 3, generator=g).to(device)
+    z = -0.3 - 0.1 * front[:, 2]
+    # the view mirrors x and y
+    scene["means3D"][:120, 0] = (0.5 * side - 4.0 - 8.0 * front[:, 0].round()) * pixel * (4.0 + z) / 4.0
+    scene["means3D"][:120, 1] = (0.5 * side - 16.0 * front[:, 1]) * pixel * (4.0 + z) / 4.0
+    scene["means3D"][:120, 2] = z
+    scene["scales"][:120] = pixel
+    scene["opacities"][:120] = 0.99
+    out = gpu_forward(scene, options())
+    ends = out["res"].n_contrib.view(side, side)[:16, :8]
+    print(f"[ends] {pixels} {int(ends.min())} {int(ends.max())} of "
+          f"{int(out['bins'].ranges[0, 1] - out['bins'].ranges[0, 0])}", flush=True)
+    assert int(ends.min()) <= 128 and int(ends.max()) > 4 * 128
+    _assert_close(*_sums(scene, out, out["res"].alpha, out["res"].n_contrib))
+    _check_backward(scene)
 
 
 @pytest.mark.gpu
