@@ -799,6 +799,7 @@ def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torc
         words = max(int(lib.gs_band_store_words(P)), 1)
         spans.append(("band_store", i32, (words,), 4 * words))
     arena = StateArena(spans, device)
+    base, offset = arena.buffer.data_ptr(), arena.offset
     radii = torch.empty((P,), dtype=i32, device=device)
     proj_2d = torch.empty((P, 2), dtype=f32, device=device)
     conic_2d = torch.empty((P, 3), dtype=f32, device=device)
@@ -806,9 +807,9 @@ def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torc
     pre = ArenaPreprocessOutputs.within(arena, radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode)
     copies = []
     tanfovx, tanfovy = float(inputs.tan_fovx), float(inputs.tan_fovy)
-    radii_at, records_at, tiles_at = radii.data_ptr(), arena.address("records"), arena.address("tiles_touched")
-    coverage_at, depths_at, inv_at = arena.address("coverage"), arena.address("depths"), conic_2d_inv.data_ptr()
-    scan_at, info_at = arena.address("scan_state"), arena.address("info")
+    radii_at, records_at, tiles_at = radii.data_ptr(), base + offset("records"), base + offset("tiles_touched")
+    coverage_at, depths_at, inv_at = base + offset("coverage"), base + offset("depths"), conic_2d_inv.data_ptr()
+    scan_at, info_at = base + offset("scan_state"), base + offset("info")
     lib.call(
         "gs_preprocess_fwd", P, K, int(inputs.degree), _address(inputs.means3d, copies),
         _address(inputs.scales, copies) if has_sr else None, _address(inputs.rotations, copies, True) if has_sr else None,
@@ -816,8 +817,8 @@ def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torc
         None if has_colors else _address(sh, copies), _address(colors, copies) if has_colors else None, _address(inputs.viewmatrix, copies),
         _address(inputs.projmatrix, copies), _address(inputs.campos, copies), tanfovx, tanfovy, _focal(W, tanfovx), _focal(H, tanfovy),
         W, H, coverage_mode, float(inputs.filter_variance), radii_at, depths_at, proj_2d.data_ptr(),
-        conic_2d.data_ptr(), inv_at, tiles_at, coverage_at, records_at, arena.address("clamped"),
-        pre.address("band_store"), words if sized else 0, scan_at, scan_bytes, stream)
+        conic_2d.data_ptr(), inv_at, tiles_at, coverage_at, records_at, base + offset("clamped"),
+        base + offset("band_store") if sized else None, words if sized else 0, scan_at, scan_bytes, stream)
     offsets = torch.empty((P,), dtype=i32, device=device)
     lib.call("gs_scan_tiles_onepass", P, tiles_at, offsets.data_ptr(), info_at, scan_at, scan_bytes, int(sized),
              SCAN_SPIN_LIMIT, stream)
@@ -838,12 +839,12 @@ def _forward_arena(inputs: RasterInputs, options: ExecutionOptions, device: torc
         lib.call("gs_readback_bin_packed", info_at, slot.address, slot.next_seq(), P, radii_at, records_at, inv_at,
                  coverage_at, depths_at, offsets.data_ptr(), W, H, coverage_mode,
                  DEPTH_TILE_MIN_PAIRS_PER_GAUSSIAN if mode == "warp_depth_stable_tile" else 0, capacity,
-                 ws.data_ptr(), ws_bytes, arena.address("ranges"), point_list.data_ptr(), background,
+                 ws.data_ptr(), ws_bytes, base + offset("ranges"), point_list.data_ptr(), background,
                  0 if flow else int(compute_depth), None if flow else color.data_ptr(),
                  None if flow else depth.data_ptr(), None if flow else alpha.data_ptr(),
-                 None if flow else arena.address("n_contrib"), None if flow else _lib.ptr(grad_gauss),
+                 None if flow else base + offset("n_contrib"), None if flow else _lib.ptr(grad_gauss),
                  0 if flow or grad_gauss is None else grad_gauss.numel(), None, result,
-                 None if flow else arena.address("tile_order"), stream)
+                 None if flow else base + offset("tile_order"), stream)
         R = validate_pair_count(result[0])
         _workspace.note_pairs(device, R)
         if result[4]:

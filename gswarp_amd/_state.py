@@ -133,8 +133,8 @@ class StateArena:
             at += (nbytes + 255) & ~255
         self.buffer = torch.empty((at,), dtype=torch.uint8, device=device)
 
-    def address(self, name: str) -> int:
-        return self.buffer.data_ptr() + self.spans[name][0]
+    def offset(self, name: str) -> int:
+        return self.spans[name][0]
 
     def view(self, name: str) -> torch.Tensor:
         at, dtype, shape, nbytes = self.spans[name]
@@ -150,7 +150,10 @@ def _arena_field(name: str) -> property:
         return self.own[name]
 
     def put(self, value):
-        self.own[name] = value
+        try:
+            self.own[name] = value
+        except AttributeError:  # the dataclass's constructor, which gives every array
+            self.arena, self.own = None, {name: value}
 
     return property(get, put)
 
@@ -165,15 +168,12 @@ class _InArena:
     __slots__ = ()
     plain: type
 
-    def __new__(cls, *args, **kwargs):
-        self = super().__new__(cls)
-        self.arena, self.own = None, {}
-        return self
-
     def address(self, name: str) -> int | None:
-        if self.arena is None or name in self.own or name not in self.arena.spans:
-            return super().address(name)
-        return self.arena.address(name)
+        if name not in self.own and self.arena is not None:
+            span = self.arena.spans.get(name)
+            if span is not None:
+                return self.arena.buffer.data_ptr() + span[0]
+        return super().address(name)
 
     def _values(self) -> dict:
         return {f.name: getattr(self, f.name) for f in fields(self)}
@@ -201,8 +201,8 @@ class ArenaPreprocessOutputs(_InArena, PreprocessOutputs):
 
     @classmethod
     def within(cls, arena: StateArena, radii, proj_2d, conic_2d, conic_2d_inv, coverage_mode: int):
-        self = cls.__new__(cls)
-        self.arena = arena
+        self = object.__new__(cls)
+        self.arena, self.own = arena, {}
         self.radii, self.proj_2d, self.conic_2d, self.conic_2d_inv = radii, proj_2d, conic_2d, conic_2d_inv
         self.coverage_mode = coverage_mode
         self.geom = None
@@ -221,8 +221,8 @@ class ArenaBinningState(_InArena, BinningState):
     @classmethod
     def within(cls, arena: StateArena, grid_x: int, grid_y: int, point_list, num_rendered: int, key_layout: KeyLayout,
                rendered: bool):
-        self = cls.__new__(cls)
-        self.arena = arena
+        self = object.__new__(cls)
+        self.arena, self.own = arena, {}
         self.grid_x, self.grid_y = grid_x, grid_y
         self.point_list, self.num_rendered, self.key_layout = point_list, num_rendered, key_layout
         self.sorted_keys = self.buffer = None
@@ -247,8 +247,8 @@ class ArenaForwardState(_InArena, ForwardState):
 
     @classmethod
     def within(cls, arena: StateArena, preprocess: PreprocessOutputs, binning: BinningState, grad_gauss):
-        self = cls.__new__(cls)
-        self.arena = arena
+        self = object.__new__(cls)
+        self.arena, self.own = arena, {}
         self.preprocess, self.binning, self.grad_gauss = preprocess, binning, grad_gauss
         return self
 
