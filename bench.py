@@ -210,8 +210,9 @@ def read_traffic(stage: str, config: int = 2):
 
 
 def read_valu_insts(stage: str, config: int = 2):
-    """VALU wave instructions per launch of a stage's kernel (the variant with the
-    most dispatches) from the committed SQ counter summary, if present."""
+    """VALU wave instructions of a stage's kernels per iteration (those with the
+    most dispatches: the variant that the workload takes, or the launches of a
+    stage of several) from the committed SQ counter summary, if present."""
     path = profile_path("sq_counters", config)
     if not path.exists():
         return None
@@ -234,6 +235,8 @@ def read_valu_insts(stage: str, config: int = 2):
             continue
         if best is None or dispatches > best[0]:
             best = (dispatches, insts)
+        elif dispatches == best[0]:
+            best = (dispatches, best[1] + insts)
     return None if best is None else best[1]
 
 
@@ -295,7 +298,11 @@ STAGE_OF_KERNEL = (
     ("gs::tile_ranges_kernel", "ranges"),
     ("gs::tile_ranges_u32_kernel", "ranges"),
     ("gs::render_fwd_kernel", "render"),
+    ("gs::render_fwd_block_kernel", "render"),
     ("gs::render_bwd_kernel", "render_bwd"),
+    ("gs::slice_walk_kernel", "render_bwd"),
+    ("gs::render_bwd_compose_kernel", "render_bwd"),
+    ("gs::render_bwd_segments_kernel", "render_bwd"),
     ("gs::render_bwd_whole_kernel", "render_bwd"),
     ("gs::preprocess_bwd_kernel", "preprocess_bwd"),
     ("gs::bucket_depth_keys_kernel", "depth_sort"),
