@@ -148,9 +148,9 @@ __device__ __forceinline__ void flush_slot(const float* slot, int gid, int lane,
 // lane 60 sum v dx^2 (2), lane 5 sum v dx (0) and lane 13 sum v dx dy (3).
 //
 // The kernel is bound by its LDS traffic about as much as by VALU issue (1M
-// Gaussians, 1080p: LDS active 1.52e8 of 2.4e8 CU cycles).  A second LDS stage
+// Gaussians, 1080p: LDS active for half of the CUs' cycles).  A second LDS stage
 // instead of the DPP steps (three stores a visit and a float4 read of them at
-// the next visit) issued 2.28e8 vector instructions to these 2.4e8, but left
+// the next visit) issued 2.29e8 vector instructions to these 2.35e8, but left
 // the LDS active 1.52e8 cycles to these 1.15e8: fwd+bwd 941 us to 905.
 constexpr int kColRawFloats = 7 * 64;
 
@@ -163,8 +163,9 @@ __device__ __forceinline__ int col_raw_offset(int lane) {
 // this ^ 1.  Odd components start with the upper half: 16 lanes (two
 // components) are served at once, and their groups lie 64 floats apart, so
 // with both components reading the same half every access met two lanes on
-// each of half the banks.  1M Gaussians, 1080p: LDS conflict cycles 3.1e7 ->
-// 0.6e7 of 1.8e8 active ones, fwd+bwd 963 -> 947 us.
+// each of half the banks.  1M Gaussians, 1080p: LDS conflict cycles 3.1e7 of
+// 1.8e8 active ones -> 0 (0.6e7 while the second LDS stage was there), fwd+bwd
+// 963 -> 947 us.
 __device__ __forceinline__ int col_group_index(int lane) {
   const int group = lane >> 3;
   return (group == 7 ? 0 : group) * 16 + (lane & 7) * 2 + (group & 1);
@@ -706,8 +707,8 @@ __device__ __forceinline__ void render_bwd_tiles(const RenderBwdParams& p) {
     render_bwd_slice<kDepth, 2, 1, false>(p, tile, quadrant, s_rec, s_slot);
 }
 
-// The halves and quadrants need 72 VGPRs, seven waves per SIMD (the bound
-// keeps them at six or more); the whole-tile walk needs more.
+// The halves and quadrants need 69 VGPRs (65 without depth), seven waves per
+// SIMD (the bound keeps them at six or more); the whole-tile walk 101 (95).
 template <bool kDepth>
 __global__ __launch_bounds__(64, 6) void render_bwd_kernel(RenderBwdParams p) {
   render_bwd_tiles<kDepth, false>(p);
@@ -720,12 +721,15 @@ __global__ __launch_bounds__(64) void render_bwd_whole_kernel(RenderBwdParams p)
 
 // The walk in segments.  On images of few tiles the slices of render_bwd_tiles
 // leave most of the chip idle, and the kernel lasts as long as its longest
-// serial walk (about 0.25 us an entry).  Here the walk of a slice (quadrants,
-// kPix 1, or halves, kPix 2) of L entries is cut into min(max_segments,
-// ceil(L / kSegmentEntries)) segments of equal length, each walked by a wave
-// of its own, after a first launch has walked every segment but the front
-// ones for its map (SegmentMode).  slice_walk_kernel finds every slice's L,
-// so that the waves of segments that do not exist return on one load.
+// serial walk (0.13 us an entry in quadrants, 0.25 in halves).  Here the walk
+// of a slice (quadrants, kPix 1, or halves, kPix 2) of L entries is cut into
+// segments of one length:
+// L over min(max_segments, ceil(L / kSegmentEntries)), rounded up to whole
+// batches of 64 (up to the cap, segments of 128 and a shorter one; with a cap of
+// 32, 4096 entries are 32 segments of 128 and 4097 are 22 of 192).  Each is
+// walked by a wave of its own, after a first launch has walked every segment
+// but the front ones for its map (SegmentMode).  slice_walk_kernel finds every
+// slice's L, so that the waves of segments that do not exist return on one load.
 //
 // Kernel times of the three launches against the unsegmented walk, us:
 // 1M Gaussians on 640x640 (4.6k entries on a few tiles) 1605 -> 190, 262k on

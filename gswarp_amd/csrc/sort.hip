@@ -1,8 +1,8 @@
 // Stable LSD radix sort of uint32 or uint64 keys (optionally with int32
 // values) for gfx950, on a bit field [lo_bit, lo_bit + key_bits) of the key.
 //
-// Per digit pass (reduce-then-scan; digits of at most 8 bits, or 9 (Plan), the
-// field split evenly over ceil(bits / 8) passes):
+// Per digit pass (reduce-then-scan; the field split evenly over as many passes
+// as digits of the plan's width, 8 bits or 9, need):
 //   1. upsweep:   each block of 2048 to 8192 elements (Plan) counts its digits -> hist[digit][block].
 //   2. rowscan:   one workgroup per digit scans hist[digit][*] across blocks
 //                 (exclusive) and records the digit total.

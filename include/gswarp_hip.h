@@ -515,9 +515,9 @@ int gs_render_bwd(int32_t image_width, int32_t image_height, int32_t num_points,
 
 /*
  * gs_render_bwd with a workspace (8-byte aligned, gs_render_bwd_workspace_bytes
- * bytes; NULL, or 0 bytes asked: gs_render_bwd itself) in which images of few
- * tiles have their walks cut into segments that run side by side.  The sums
- * differ only by rounding.
+ * bytes for the same sizes, of any content; NULL, or 0 bytes asked:
+ * gs_render_bwd itself) in which images of few tiles have their walks cut into
+ * segments that run side by side.  The sums differ only by rounding.
  * Replaces: backward_ops.py:183-290 with backward_kernels.py:539-707.
  */
 size_t gs_render_bwd_workspace_bytes(int32_t image_width, int32_t image_height, int32_t num_points,
