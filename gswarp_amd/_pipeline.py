@@ -922,7 +922,7 @@ def backward(inputs: RasterInputs, radii: torch.Tensor, alpha: torch.Tensor, gra
             background = inputs.background.to(device)  # held: a copy on the device is freed with its last reference
             with _stage("render_bwd"):
                 lib.call("gs_render_bwd_ws", W, H, P, bins.num_rendered, bins.address("ranges"),
-                         bins.address("point_list"), records_at, _address(background, copies),
+                         bins.point_list.data_ptr(), records_at, _address(background, copies),
                          _address(alpha, copies), n_contrib_at, _address_or_none(grad_color, copies),
                          _address_or_none(grad_depth, copies), _address_or_none(grad_alpha, copies),
                          int(bool(options.compute_depth)), grad_gauss_at, bins.address("tile_order"), _lib.ptr(ws),
